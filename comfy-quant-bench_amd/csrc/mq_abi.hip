@@ -563,9 +563,10 @@ int mq_linear_w4_group(const void* x, int x_dtype, int64_t ldx, int hblock, int 
                        bias_dtype, y, y_dtype, ldy, M, N, K, base + w.split, workspace_bytes - w.split, &a);
     if (rc) return rc == kEmpty ? MQ_OK : rc;
     const WKind wk = wz ? WKind::U4Asym : WKind::I4Sym;
-    a.atile = 1;   // the codes in 16-row tiles wherever the wide kernel reads them
-    a.atile = gemm_runs_wide(a, wk, Epi::GroupScale);
-    if (a.wtile && !a.atile) {
+    a.atile = 1;   // the codes in 16-row tiles wherever the wide or few-row kernel reads them
+    const bool wide = gemm_runs_wide(a, wk, Epi::GroupScale);
+    a.atile = wide || gemm_runs_few(a, wk, Epi::GroupScale);
+    if (a.wtile && !wide) {
         set_error("linear_w4_group: expanded 4-bit weights are read by the wide kernel only (M > 4, operands under "
                   "2 GiB); pass the packed weights");
         return MQ_EUNSUPPORTED;
@@ -592,8 +593,8 @@ int mq_linear_rowscale(const void* x, int x_dtype, int64_t ldx, int hblock, int 
                        qw, ldw, wbits, ws, bias, bias_dtype, y, y_dtype, ldy, M, N, K, base + w.split,
                        workspace_bytes - w.split, &a, &wk);
     if (rc) return rc == kEmpty ? MQ_OK : rc;
-    a.atile = 1;   // the codes in 16-row tiles wherever the wide kernel reads them
-    a.atile = gemm_runs_wide(a, wk, Epi::RowScale);
+    a.atile = 1;   // the codes in 16-row tiles wherever the wide or few-row kernel reads them
+    a.atile = gemm_runs_wide(a, wk, Epi::RowScale) || gemm_runs_few(a, wk, Epi::RowScale);
     if (swiglu == MQ_SWIGLU_NONE && gemv_quantizes_row(a, wk, Epi::RowScale))
         return launch_fused_row(a, wk, Epi::RowScale, x, x_dtype, ldx, hblock, act_bits, MQ_Q_BYTES, base, stream);
     rc = quantize_into(x, x_dtype, ldx, hblock, act_bits, swiglu, MQ_Q_BYTES, a.atile, M, K, base, stream);

@@ -1,4 +1,7 @@
-// Quantized GEMMs on gfx950 int8 MFMA (v_mfma_i32_32x32x32_i8) with LDS-staged tiles.
+// Quantized GEMMs on gfx950 int8 MFMA (v_mfma_i32_32x32x32_i8) with LDS-staged tiles, and the dispatch
+// over all GEMM kernels (launch_gemm). This kernel serves the parity entries up to 128 rows and what
+// the others do not take: K < 192, activation layout 1 above 128 rows, zero-point or scale rows that
+// are not aligned for the wide kernel, operands past its 32-bit offsets.
 //
 // Workgroup tile 128 (M) x 128 (N) x 64 (K = one weight group per k-step), 4 wavefronts in a
 // 2 x 2 grid, each owning a 64 x 64 output tile made of 2 x 2 MFMA 32x32 tiles. Global loads of
@@ -271,8 +274,24 @@ bool gemv_quantizes_row(const GemmArgs& a, WKind wk, Epi epi) {
     return runs_gemv(a, wk, epi) && a.M == 1 && a.K <= 4096 && (epi == Epi::GroupScale || epi == Epi::RowScale);
 }
 
+bool gemm_runs_few(const GemmArgs& a, WKind wk, Epi epi) {
+    if (runs_gemv(a, wk, epi) || a.M > 128 || a.K % 64 || a.K > 65536) return false;   // 16 * v int4 sums fit int32
+    // 32-bit lane offsets over 64 weight rows and 128 activation rows
+    constexpr int64_t kMaxStride = int64_t(1) << 23;
+    if (a.lda > kMaxStride || a.ldw > kMaxStride || a.ldws > kMaxStride || a.ldwz > kMaxStride) return false;
+    if (epi == Epi::GroupScale) return wk != WKind::I8 && !a.wtile;   // (expanded weights: the wide kernel's)
+    if (epi != Epi::RowScale || wk == WKind::U4Asym) return false;
+    // Every kernel sums int32 exactly, so the quicker one takes the product. Many columns and rows:
+    // the wide kernel's 128 x 128 tiles share each operand over more products than the few-row
+    // kernel's 32 or 64 columns do (W8A8 linears, K = 3072, few-row / wide: M = 128 N = 8192 16.1 / 19.1,
+    // N = 12288 21.1 / 19.6, N = 18432 31.2 / 20.5 us; M = 48 N = 18432 19.0 / 19.8 us).
+    const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256, blocks = (a.N + 15) / 16;
+    // (the wide kernel takes so few rows with weights in 16-row tiles only)
+    return !a.wtile || (!(blocks > 2 * cus && a.M > 80) && !(blocks > 4 * cus && a.M > 48));
+}
+
 bool gemm_runs_wide(const GemmArgs& a, WKind wk, Epi epi) {
-    if (runs_gemv(a, wk, epi)) return false;
+    if (runs_gemv(a, wk, epi) || gemm_runs_few(a, wk, epi)) return false;
     // The 256 x 256-tile kernel addresses each operand with 32-bit buffer offsets.
     // (4-bit weights with wtile set come expanded to int8 tiles, K bytes per row)
     const int64_t wbytes = wk == WKind::I8 || a.wtile ? a.K : a.K / 2;
@@ -293,8 +312,8 @@ bool gemm_runs_wide(const GemmArgs& a, WKind wk, Epi epi) {
 
 int launch_gemm(const GemmArgs& a, WKind wk, Epi epi, hipStream_t stream) {
     if (a.M == 0 || a.N == 0) return 0;
-    if (a.atile && !gemm_runs_wide(a, wk, epi)) {
-        set_error("gemm: activation codes in 16-row tiles are read by the wide kernel only");
+    if (a.atile && !gemm_runs_wide(a, wk, epi) && !gemm_runs_few(a, wk, epi)) {
+        set_error("gemm: activation codes in 16-row tiles are read by the wide and few-row kernels only");
         return -2;
     }
     if (a.wtile && wk != WKind::I8 && !gemm_runs_wide(a, wk, epi)) {
@@ -305,6 +324,7 @@ int launch_gemm(const GemmArgs& a, WKind wk, Epi epi, hipStream_t stream) {
     // a few rows: HBM-bound, served by the dot4 kernel (activation rows staged in LDS); its parity
     // entries (exact group partials, full-K sums) run the same kernel
     if (runs_gemv(a, wk, epi)) return launch_gemv(a, wk, epi, stream);
+    if (gemm_runs_few(a, wk, epi)) return launch_gemm_few(a, wk, epi, stream);
     if (gemm_runs_wide(a, wk, epi)) {
         GemmArgs w = a;
         w.ksplit = 1;

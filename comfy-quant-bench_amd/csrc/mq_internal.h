@@ -151,6 +151,11 @@ int launch_gemv(const GemmArgs& a, WKind wk, Epi epi, hipStream_t stream);
 // the rotate+quantize kernel's arithmetic, in the same launch.
 bool gemv_quantizes_row(const GemmArgs& a, WKind wk, Epi epi);
 
+// 5 <= M <= 128 rows, GroupScale / RowScale (mq_gemm_few.hip); whether launch_gemm runs these
+// arguments' product there (it reads qa in rows or in 16-row tiles).
+int launch_gemm_few(const GemmArgs& a, WKind wk, Epi epi, hipStream_t stream);
+bool gemm_runs_few(const GemmArgs& a, WKind wk, Epi epi);
+
 // 256 x 256-tile kernel for large M (mq_gemm_wide.hip).
 int launch_gemm_wide(const GemmArgs& a, WKind wk, Epi epi, hipStream_t stream);
 
