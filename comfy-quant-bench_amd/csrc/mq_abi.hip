@@ -220,9 +220,9 @@ int mq_decode_w4a8_codebook(const void* qdata, int64_t ldq, const void* s_rel, i
                                        static_cast<hipStream_t>(stream));
 }
 
-int mq_quantize_weight(const void* w, int dtype, int64_t N, int64_t K, int64_t ldw, int hblock, int format,
-                       void* q, int64_t ldq, void* scale, int64_t ld_scale, void* zero, int64_t ld_zero,
-                       void* stream) {
+int mq_quantize_weight_checked(const void* w, int dtype, int64_t N, int64_t K, int64_t ldw, int hblock, int format,
+                               void* q, int64_t ldq, void* scale, int64_t ld_scale, void* zero, int64_t ld_zero,
+                               int32_t* nonfinite, void* stream) {
     clear_error();
     MQ_REQUIRE(dtype >= MQ_DT_BF16 && dtype <= MQ_DT_F32, "quantize_weight: unknown dtype %d", dtype);
     MQ_REQUIRE(format >= MQ_WFMT_U4_ASYM_G64 && format <= MQ_WFMT_I8_ROW, "quantize_weight: unknown format %d", format);
@@ -252,8 +252,15 @@ int mq_quantize_weight(const void* w, int dtype, int64_t N, int64_t K, int64_t l
     }
     if (format == MQ_WFMT_U4_ASYM_G64)
         MQ_REQUIRE(zero && ld_zero >= (K / 64 + 1) / 2, "quantize_weight: zero needs ld_zero >= ceil(K/128)");
+    MQ_REQUIRE(aligned(nonfinite, 4), "quantize_weight: nonfinite must be 4-byte aligned");
     return launch_quantize_weight(w, dtype, N, K, ldw, hblock, format, q, ldq, scale, ld_scale, zero, ld_zero,
-                                  static_cast<hipStream_t>(stream));
+                                  nonfinite, static_cast<hipStream_t>(stream));
+}
+
+int mq_quantize_weight(const void* w, int dtype, int64_t N, int64_t K, int64_t ldw, int hblock, int format, void* q,
+                       int64_t ldq, void* scale, int64_t ld_scale, void* zero, int64_t ld_zero, void* stream) {
+    return mq_quantize_weight_checked(w, dtype, N, K, ldw, hblock, format, q, ldq, scale, ld_scale, zero, ld_zero,
+                                      nullptr, stream);
 }
 
 int mq_tile_weight_i8(const int8_t* w, int64_t ldw, int64_t N, int64_t K, int8_t* out, void* stream) {

@@ -48,7 +48,7 @@ int launch_decode_w4a8_codebook(const uint8_t* qdata, int64_t ldq, const uint8_t
 // --- offline weight quantizer (mq_wquant.hip); dtype / format are MQ_DT_* / MQ_WFMT_*
 int launch_quantize_weight(const void* w, int dtype, int64_t N, int64_t K, int64_t ldw, int hblock, int format,
                            void* q, int64_t ldq, void* scale, int64_t ld_scale, void* zero, int64_t ld_zero,
-                           hipStream_t stream);
+                           int* nonfinite, hipStream_t stream);
 
 // int8 weights [N, K] into the 16-row tile layout of GemmArgs::wtile (mq_wquant.hip)
 int launch_tile_weight_i8(const uint8_t* w, int64_t ldw, int64_t N, int64_t K, uint8_t* out, hipStream_t stream);

@@ -1,188 +1,296 @@
 // Offline weight quantizer (the converter side of the path): rotate each weight row by H_hblock and
 // quantize it to one of the GEMMs' weight formats.
 //
-// One 256-thread workgroup per weight row. The row is staged in LDS as fp32 (K <= 32768, 128 KB),
-// rotated in place by the pinned radix-4 FWHT (experiments/qwen21-kernel/kernels/g64_quant.cu:68-86:
-// stages with element strides 1, 4, 16, 64, h = 0.5f * (((x0 + x1) + x2) + x3), y_i = h - x_{3-i},
-// the same fp32 operations as the activation kernel and the torch / numpy quantizers), then
-// quantized with IEEE divisions:
-//   U4_ASYM_G64  lo = min(min w, 0), hi = max(max w, 0), s = fp16((hi - lo) / 15),
+// The rotation is the activation quantizer's (mq_rotate.h: one wavefront per 1024-column chunk, each
+// lane 16 consecutive columns, the pinned radix-4 FWHT of
+// experiments/qwen21-kernel/kernels/g64_quant.cu:68-86 in registers and an LDS transpose). The group
+// formats need nothing across chunks (a 64-column group is four lanes of one 16-lane row), so every
+// wave takes one chunk of one row and nothing waits at a barrier; the row formats give a row to the
+// four waves of a workgroup, NCH chunks each, which combine the row's maximum through LDS. With
+////   U4_ASYM_G64  lo = min(min w, 0), hi = max(max w, 0), s = fp16((hi - lo) / 15),
 //                z = clamp(rne(-lo / s), 0, 15), q = clamp(rne(w / s) + z, 0, 15); s = 0 -> q = z = 0
 //   I4_SYM_G64   s = fp16(max |w| / 7), q = clamp(rne(w / s), -7, 7); s = 0 -> q = 0
 //   I4_ROW       s = max(max |w|, 1e-10) / 7,   q = clamp(rne(w / s), -7, 7)
 //   I8_ROW       s = max(max |w|, 1e-10) / 127, q = clamp(rne(w / s), -127, 127)
-// (the group formats are the configs' schemes, with the min / max code choice of
-// custom_nodes/comfy-lowbit-loader/formats.py:131-149 and the symmetric form of
+// where w is the rotated weight (the group formats are the configs' schemes, with the min / max code
+// choice of custom_nodes/comfy-lowbit-loader/formats.py:131-149 and the symmetric form of
 // tools/svdquant_probe.py:105-115; the row formats are tools/gptq_w4a4.py:197-203 and
-// tools/_formats.py:128-167). The quantizer runs once per weight, so it favours a simple exact
-// structure over speed: the row is read once from HBM and each output byte written once.
+// tools/_formats.py:128-167). Scales and zero-points come from IEEE divisions. Codes take the
+// activation quantizer's product with the reciprocal and its exact division wherever that product
+// lies near a half-integer (quant16's argument: |w / s| < 128, here at most 127 or, for an fp16 scale
+// rounded down in its subnormal range, 23), so they are the IEEE quotient's codes.
+//
+// What bounds it: HBM, 2.5 bytes per bf16 weight. At N = 12288, K = 3072 (96 MB): 26.5 us; one
+// workgroup per row with the row in LDS, a barrier per butterfly stage, one thread per group and
+// an IEEE division per weight took 142 us.
 #include "mq_device.h"
 #include <algorithm>
 #include "mq_internal.h"
+#include "mq_rotate.h"
 
 #pragma clang fp contract(off)
 
 namespace mq {
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int kMaxK = 32768;
-constexpr int kMaxGroups = kMaxK / 64;
-
-template <int DT>
-__device__ __forceinline__ float load_w(const void* w, int64_t i) {
-    if constexpr (DT == 0) return __uint_as_float(static_cast<uint32_t>(static_cast<const uint16_t*>(w)[i]) << 16);
-    else if constexpr (DT == 1) return static_cast<float>(static_cast<const _Float16*>(w)[i]);
-    else return static_cast<const float*>(w)[i];
-}
+constexpr int kWaves = 4;   // wavefronts per workgroup
 
 __device__ __forceinline__ float clampf(float v, float lo, float hi) { return __builtin_fminf(__builtin_fmaxf(v, lo), hi); }
 
-// Maximum over the workgroup (every thread gets it); red holds one float per wavefront.
-__device__ __forceinline__ float block_max(float v, float* red) {
-    v = wave_max(v);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    float m = red[0];
+// 16 consecutive weights of type DT at element i of w, as fp32; vec: 16-byte loads (the host has
+// checked the base and the row stride), else element by element.
+template <int DT>
+__device__ __forceinline__ void load16(const void* w, int64_t i, bool vec, float (&v)[16]) {
+    if constexpr (DT == kDtF32) {
+        const float* p = static_cast<const float*>(w) + i;
+        if (vec) {
 #pragma unroll
-    for (int i = 1; i < kThreads / 64; ++i) m = __builtin_fmaxf(m, red[i]);
-    return m;
-}
-
-template <int DT, int FMT>
-__global__ void __launch_bounds__(kThreads)
-wquant_kernel(const void* __restrict__ w, int64_t ldw, int K, int hblock, uint8_t* __restrict__ q, int64_t ldq,
-              void* __restrict__ scale, int64_t ld_scale, uint8_t* __restrict__ zero, int64_t ld_zero) {
-    extern __shared__ float row[];                    // K fp32 values
-    __shared__ float gs[kMaxGroups];                  // per-group scale (fp32 value of the fp16)
-    __shared__ float gz[kMaxGroups];                  // per-group zero-point
-    __shared__ float red[kThreads / 64];
-    const int tid = threadIdx.x;
-    const int64_t n = blockIdx.x;
-
-    for (int i = tid; i < K; i += kThreads) row[i] = load_w<DT>(w, n * ldw + i);
-    __syncthreads();
-
-    // pinned radix-4 FWHT: butterfly b of a stage with stride st has x_j at i0 + j st,
-    // i0 = (b / st) 4 st + b % st (4 st divides hblock, so butterflies never straddle blocks)
-    for (int st = 1; st < hblock; st *= 4) {
-        for (int b = tid; b < K / 4; b += kThreads) {
-            const int i0 = (b / st) * 4 * st + b % st;
-            const float x0 = row[i0], x1 = row[i0 + st], x2 = row[i0 + 2 * st], x3 = row[i0 + 3 * st];
-            const float h = 0.5f * (((x0 + x1) + x2) + x3);
-            row[i0] = h - x3;
-            row[i0 + st] = h - x2;
-            row[i0 + 2 * st] = h - x1;
-            row[i0 + 3 * st] = h - x0;
-        }
-        __syncthreads();
-    }
-
-    if constexpr (FMT == 0 || FMT == 1) {
-        const int G = K / 64;
-        uint16_t* s16 = static_cast<uint16_t*>(scale) + n * ld_scale;
-        for (int g = tid; g < G; g += kThreads) {
-            const float* v = row + 64 * g;
-            float s;
-            if constexpr (FMT == 0) {
-                float mn = v[0], mx = v[0];
-                for (int e = 1; e < 64; ++e) {
-                    mn = __builtin_fminf(mn, v[e]);
-                    mx = __builtin_fmaxf(mx, v[e]);
-                }
-                const float lo = __builtin_fminf(mn, 0.0f), hi = __builtin_fmaxf(mx, 0.0f);
-                const _Float16 h = static_cast<_Float16>((hi - lo) / 15.0f);
-                s = static_cast<float>(h);
-                gz[g] = s == 0.0f ? 0.0f : clampf(__builtin_rintf(-lo / s), 0.0f, 15.0f);
-                s16[g] = __builtin_bit_cast(uint16_t, h);
-            } else {
-                float am = 0.0f;
-                for (int e = 0; e < 64; ++e) am = __builtin_fmaxf(am, __builtin_fabsf(v[e]));
-                const _Float16 h = static_cast<_Float16>(am / 7.0f);
-                s = static_cast<float>(h);
-                s16[g] = __builtin_bit_cast(uint16_t, h);
+            for (int j = 0; j < 4; ++j) {
+                const float4 f = *reinterpret_cast<const float4*>(p + 4 * j);
+                v[4 * j] = f.x;
+                v[4 * j + 1] = f.y;
+                v[4 * j + 2] = f.z;
+                v[4 * j + 3] = f.w;
             }
-            gs[g] = s;
-        }
-        __syncthreads();
-        // eight consecutive codes per thread step: one packed dword
-        uint8_t* qr = q + n * ldq;
-        for (int i = 8 * tid; i < K; i += 8 * kThreads) {
-            const int g = i / 64;
-            const float s = gs[g];
-            uint32_t word = 0;
+        } else {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                int c = 0;
-                if (s != 0.0f) {
-                    if constexpr (FMT == 0) c = static_cast<int>(clampf(__builtin_rintf(row[i + e] / s) + gz[g], 0.0f, 15.0f));
-                    else c = static_cast<int>(clampf(__builtin_rintf(row[i + e] / s), -7.0f, 7.0f));
-                }
-                word |= (static_cast<uint32_t>(c) & 0xfu) << (4 * e);
-            }
-            *reinterpret_cast<uint32_t*>(qr + i / 2) = word;
-        }
-        if constexpr (FMT == 0) {
-            uint8_t* zr = zero + n * ld_zero;
-            for (int j = tid; j < (G + 1) / 2; j += kThreads) {
-                const uint32_t z0 = static_cast<uint32_t>(gz[2 * j]);
-                const uint32_t z1 = 2 * j + 1 < G ? static_cast<uint32_t>(gz[2 * j + 1]) : 0u;
-                zr[j] = static_cast<uint8_t>(z0 | (z1 << 4));
-            }
+            for (int j = 0; j < 16; ++j) v[j] = p[j];
         }
     } else {
-        constexpr float L = FMT == 2 ? 7.0f : 127.0f;
-        float am = 0.0f;
-        for (int i = tid; i < K; i += kThreads) am = __builtin_fmaxf(am, __builtin_fabsf(row[i]));
-        am = block_max(am, red);
-        const float s = __builtin_fmaxf(am, 1e-10f) / L;
-        if (tid == 0) static_cast<float*>(scale)[n] = s;
-        uint8_t* qr = q + n * ldq;
-        for (int i = 8 * tid; i < K; i += 8 * kThreads) {
-            int c[8];
+        const uint16_t* p = static_cast<const uint16_t*>(w) + i;
+        uint32_t h[8];
+        if (vec) {
+            const uint4 a = *reinterpret_cast<const uint4*>(p), b = *reinterpret_cast<const uint4*>(p + 8);
+            h[0] = a.x; h[1] = a.y; h[2] = a.z; h[3] = a.w;
+            h[4] = b.x; h[5] = b.y; h[6] = b.z; h[7] = b.w;
+        } else {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) c[e] = static_cast<int>(clampf(__builtin_rintf(row[i + e] / s), -L, L));
-            if constexpr (FMT == 2) {
-                uint32_t word = 0;
+            for (int j = 0; j < 8; ++j) h[j] = p[2 * j] | static_cast<uint32_t>(p[2 * j + 1]) << 16;
+        }
 #pragma unroll
-                for (int e = 0; e < 8; ++e) word |= (static_cast<uint32_t>(c[e]) & 0xfu) << (4 * e);
-                *reinterpret_cast<uint32_t*>(qr + i / 2) = word;
-            } else {
-                uint32_t lo = 0, hi = 0;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    lo |= (static_cast<uint32_t>(c[e]) & 0xffu) << (8 * e);
-                    hi |= (static_cast<uint32_t>(c[e + 4]) & 0xffu) << (8 * e);
-                }
-                *reinterpret_cast<uint2*>(qr + i) = uint2{lo, hi};
-            }
+        for (int j = 0; j < 8; ++j) {
+            v[2 * j] = DT == kDtF16 ? f16lo(h[j]) : bf16lo(h[j]);
+            v[2 * j + 1] = DT == kDtF16 ? f16hi(h[j]) : bf16hi(h[j]);
         }
     }
+}
+
+// rotate_chunk_lds with the Hadamard block chosen at run time (wave-uniform).
+__device__ __forceinline__ void rotate(float (&v)[16], const LdsTranspose& tr, int hblock) {
+    if (hblock >= 16) {
+        stage_reg<0>(v);
+        stage_reg<2>(v);
+    }
+    if (hblock >= 64) {
+        tr(v);
+        stage_reg<0>(v);
+        if (hblock >= 256) stage_reg<2>(v);
+        tr(v);
+    }
+}
+
+// rne(v / s) of 16 weights as floats, for |v / s| < 128 and r = recip_row(s): the rounded product,
+// or the IEEE quotient's rounding where the product lies near a half-integer (quant16).
+__device__ __forceinline__ void round16(const float (&v)[16], float r, float s, float (&n)[16]) {
+    float dmax = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        n[j] = __builtin_fmaf(v[j], r, kMagic) - kMagic;
+        dmax = __builtin_fmaxf(dmax, __builtin_fabsf(__builtin_fmaf(v[j], r, -n[j])));
+    }
+    if (dmax > kTieWindow) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+            if (__builtin_fabsf(__builtin_fmaf(v[j], r, -n[j])) > kTieWindow) n[j] = __builtin_rintf(v[j] / s);
+    }
+}
+
+// 16 codes (small integers as floats) as nibbles of two dwords, or as bytes of four.
+__device__ __forceinline__ uint32_t nibbles8(const float* c) {
+    uint32_t w = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w |= (static_cast<uint32_t>(static_cast<int>(c[e])) & 0xfu) << (4 * e);
+    return w;
+}
+__device__ __forceinline__ uint32_t bytes4(const float* c) {
+    uint32_t w = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w |= (static_cast<uint32_t>(static_cast<int>(c[e])) & 0xffu) << (8 * e);
+    return w;
+}
+// 8 bytes of packed codes at p (4-byte aligned; wide: 8-byte aligned)
+__device__ __forceinline__ void store8(uint8_t* p, uint32_t lo, uint32_t hi, bool wide) {
+    if (wide) {
+        *reinterpret_cast<uint2*>(p) = uint2{lo, hi};
+    } else {
+        *reinterpret_cast<uint32_t*>(p) = lo;
+        *reinterpret_cast<uint32_t*>(p + 4) = hi;
+    }
+}
+
+// Group formats: wave u of the grid takes chunk u % chunks of row u / chunks. nonfinite (or null) is
+// set to 1 where a group's scale is not finite.
+template <int DT, int FMT>
+__global__ void __launch_bounds__(64 * kWaves)
+wquant_group_kernel(const void* __restrict__ w, int64_t ldw, int64_t N, int K, int chunks, int hblock, bool vec,
+                    uint8_t* __restrict__ q, int64_t ldq, bool wide, uint16_t* __restrict__ scale, int64_t ld_scale,
+                    uint8_t* __restrict__ zero, int64_t ld_zero, int* nonfinite) {
+    static_assert(FMT == 0 || FMT == 1, "U4_ASYM_G64, I4_SYM_G64");
+    __shared__ __attribute__((aligned(16))) float tr_lds[kWaves * kTrWave];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int seg = (lane >> 2) + 16 * (lane & 3);
+    float* tb = tr_lds + wave * kTrWave + (lane & 3) * kTrG;
+    const LdsTranspose tr{tb + (lane >> 2), tb + (lane >> 2) * kTrS};
+    for (int64_t unit = static_cast<int64_t>(blockIdx.x) * kWaves + wave; unit < N * chunks;
+         unit += static_cast<int64_t>(gridDim.x) * kWaves) {
+        const int64_t row = unit / chunks;
+        const int col = static_cast<int>(unit % chunks) * 1024 + 16 * seg;
+        const bool in = col < K;   // lanes past the row work on its first columns and store nothing
+        float v[16];
+        load16<DT>(w, row * ldw + (in ? col : 0), vec, v);
+        rotate(v, tr, hblock);
+
+        // the group's extremes: 16 values here, then the four lanes that differ in lane bits 2 and 3
+        float s, z = 0.0f;
+        _Float16 h;
+        if constexpr (FMT == 0) {
+            float mn = v[0], mx = v[0];
+#pragma unroll
+            for (int e = 1; e < 16; ++e) {
+                mn = __builtin_fminf(mn, v[e]);
+                mx = __builtin_fmaxf(mx, v[e]);
+            }
+            mn = __builtin_fminf(mn, dpp_mov<kRowRor4>(mn));
+            mx = __builtin_fmaxf(mx, dpp_mov<kRowRor4>(mx));
+            mn = __builtin_fminf(mn, dpp_mov<kRowRor8>(mn));
+            mx = __builtin_fmaxf(mx, dpp_mov<kRowRor8>(mx));
+            const float lo = __builtin_fminf(mn, 0.0f), hi = __builtin_fmaxf(mx, 0.0f);
+            h = static_cast<_Float16>((hi - lo) / 15.0f);
+            s = static_cast<float>(h);
+            z = s == 0.0f ? 0.0f : clampf(__builtin_rintf(-lo / s), 0.0f, 15.0f);
+        } else {
+            float am = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) am = __builtin_fmaxf(am, __builtin_fabsf(v[e]));
+            am = __builtin_fmaxf(am, dpp_mov<kRowRor4>(am));
+            am = __builtin_fmaxf(am, dpp_mov<kRowRor8>(am));
+            h = static_cast<_Float16>(am / 7.0f);
+            s = static_cast<float>(h);
+        }
+        float c[16];
+        round16(v, recip_row(s), s, c);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            c[e] = FMT == 0 ? clampf(c[e] + z, 0.0f, 15.0f) : clampf(c[e], -7.0f, 7.0f);
+            if (s == 0.0f) c[e] = 0.0f;
+        }
+        if (in) store8(q + row * ldq + col / 2, nibbles8(c), nibbles8(c + 8), wide);
+        const bool lead = in && (lane & 12) == 0;   // one lane per group, of column col
+        if (lead) {
+            scale[row * ld_scale + col / 64] = __builtin_bit_cast(uint16_t, h);
+            if (nonfinite && !(s < __builtin_inff())) *nonfinite = 1;
+        }
+        if constexpr (FMT == 0) {
+            // two groups per byte: the odd one sits 16 lanes on (absent past an odd number of groups)
+            const int zi = in ? static_cast<int>(z) : 0;
+            const int z1 = __shfl_xor(zi, 16, 64);
+            if (lead && (lane & 16) == 0) zero[row * ld_zero + col / 128] = static_cast<uint8_t>(zi | (z1 << 4));
+        }
+    }
+}
+
+// Row formats: one workgroup per row, wave i its chunks i, i + 4, ...
+template <int DT, int FMT, int NCH>
+__global__ void __launch_bounds__(64 * kWaves)
+wquant_row_kernel(const void* __restrict__ w, int64_t ldw, int K, int hblock, bool vec, uint8_t* __restrict__ q,
+                  int64_t ldq, bool wide, float* __restrict__ scale) {
+    static_assert(FMT == 2 || FMT == 3, "I4_ROW, I8_ROW");
+    __shared__ __attribute__((aligned(16))) float tr_lds[kWaves * kTrWave];
+    __shared__ float red[kWaves];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t row = blockIdx.x;
+    const int seg = (lane >> 2) + 16 * (lane & 3);
+    float* tb = tr_lds + wave * kTrWave + (lane & 3) * kTrG;
+    const LdsTranspose tr{tb + (lane >> 2), tb + (lane >> 2) * kTrS};
+    float v[NCH][16], am = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        const int col = (i * kWaves + wave) * 1024 + 16 * seg;
+        load16<DT>(w, row * ldw + (col < K ? col : 0), vec, v[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        rotate(v[i], tr, hblock);
+        if ((i * kWaves + wave) * 1024 + 16 * seg < K)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) am = __builtin_fmaxf(am, __builtin_fabsf(v[i][e]));
+    }
+    am = wave_max_nonneg(am);
+    if (lane == 0) red[wave] = am;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) am = __builtin_fmaxf(am, red[i]);
+    constexpr float L = FMT == 2 ? 7.0f : 127.0f;
+    const float s = __builtin_fmaxf(am, 1e-10f) / L, r = recip_row(s);
+    if (threadIdx.x == 0) scale[row] = s;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        const int col = (i * kWaves + wave) * 1024 + 16 * seg;
+        if (col >= K) continue;
+        float c[16];
+        round16(v[i], r, s, c);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) c[e] = clampf(c[e], -L, L);
+        if constexpr (FMT == 2) {
+            store8(q + row * ldq + col / 2, nibbles8(c), nibbles8(c + 8), wide);
+        } else if (wide) {
+            *reinterpret_cast<uint4*>(q + row * ldq + col) = uint4{bytes4(c), bytes4(c + 4), bytes4(c + 8), bytes4(c + 12)};
+        } else {
+            *reinterpret_cast<uint2*>(q + row * ldq + col) = uint2{bytes4(c), bytes4(c + 4)};
+            *reinterpret_cast<uint2*>(q + row * ldq + col + 8) = uint2{bytes4(c + 8), bytes4(c + 12)};
+        }
+    }
+}
+
+bool aligned_rows(const void* p, int64_t stride_bytes, int64_t n) {
+    return reinterpret_cast<uintptr_t>(p) % n == 0 && stride_bytes % n == 0;
 }
 
 template <int DT, int FMT>
 int launch_fmt(const void* w, int64_t ldw, int64_t N, int64_t K, int hblock, void* q, int64_t ldq, void* scale,
-               int64_t ld_scale, void* zero, int64_t ld_zero, hipStream_t stream) {
-    auto kern = wquant_kernel<DT, FMT>;
-    const size_t lds = static_cast<size_t>(K) * sizeof(float);
-    if (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) != hipSuccess) {
-        set_error("quantize_weight: cannot reserve %zu bytes of LDS", lds);
-        return -3;
+               int64_t ld_scale, void* zero, int64_t ld_zero, int* nonfinite, hipStream_t stream) {
+    const bool vec = aligned_rows(w, ldw * (DT == kDtF32 ? 4 : 2), 16);
+    const bool wide = aligned_rows(q, ldq, FMT == 3 ? 16 : 8);
+    const int chunks = static_cast<int>((K + 1023) / 1024);
+    auto* qb = static_cast<uint8_t*>(q);
+    if constexpr (FMT <= 1) {
+        const int64_t blocks = std::min<int64_t>((N * chunks + kWaves - 1) / kWaves, int64_t(1) << 22);
+        hipLaunchKernelGGL((wquant_group_kernel<DT, FMT>), dim3(static_cast<unsigned>(blocks)), dim3(64 * kWaves), 0,
+                           stream, w, ldw, N, static_cast<int>(K), chunks, hblock, vec, qb, ldq, wide,
+                           static_cast<uint16_t*>(scale), ld_scale, static_cast<uint8_t*>(zero), ld_zero, nonfinite);
+    } else {
+        const dim3 grid(static_cast<unsigned>(N)), block(64 * kWaves);
+        auto* sc = static_cast<float*>(scale);
+#define MQ_WQ(NCH)                                                                                            \
+    hipLaunchKernelGGL((wquant_row_kernel<DT, FMT, NCH>), grid, block, 0, stream, w, ldw, static_cast<int>(K), \
+                       hblock, vec, qb, ldq, wide, sc)
+        if (chunks <= kWaves) MQ_WQ(1);
+        else if (chunks <= 2 * kWaves) MQ_WQ(2);
+        else if (chunks <= 4 * kWaves) MQ_WQ(4);
+        else MQ_WQ(8);   // K <= 32768
+#undef MQ_WQ
     }
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(N)), dim3(kThreads), lds, stream, w, ldw, static_cast<int>(K),
-                       hblock, static_cast<uint8_t*>(q), ldq, scale, ld_scale, static_cast<uint8_t*>(zero), ld_zero);
     return launch_status("quantize_weight");
 }
 
 template <int DT>
 int launch_dt(const void* w, int64_t ldw, int64_t N, int64_t K, int hblock, int format, void* q, int64_t ldq,
-              void* scale, int64_t ld_scale, void* zero, int64_t ld_zero, hipStream_t stream) {
+              void* scale, int64_t ld_scale, void* zero, int64_t ld_zero, int* nonfinite, hipStream_t stream) {
     switch (format) {
-        case 0: return launch_fmt<DT, 0>(w, ldw, N, K, hblock, q, ldq, scale, ld_scale, zero, ld_zero, stream);
-        case 1: return launch_fmt<DT, 1>(w, ldw, N, K, hblock, q, ldq, scale, ld_scale, zero, ld_zero, stream);
-        case 2: return launch_fmt<DT, 2>(w, ldw, N, K, hblock, q, ldq, scale, ld_scale, zero, ld_zero, stream);
-        case 3: return launch_fmt<DT, 3>(w, ldw, N, K, hblock, q, ldq, scale, ld_scale, zero, ld_zero, stream);
+        case 0: return launch_fmt<DT, 0>(w, ldw, N, K, hblock, q, ldq, scale, ld_scale, zero, ld_zero, nonfinite, stream);
+        case 1: return launch_fmt<DT, 1>(w, ldw, N, K, hblock, q, ldq, scale, ld_scale, zero, ld_zero, nonfinite, stream);
+        case 2: return launch_fmt<DT, 2>(w, ldw, N, K, hblock, q, ldq, scale, ld_scale, zero, ld_zero, nonfinite, stream);
+        case 3: return launch_fmt<DT, 3>(w, ldw, N, K, hblock, q, ldq, scale, ld_scale, zero, ld_zero, nonfinite, stream);
         default: break;
     }
     set_error("quantize_weight: unknown format %d", format);
@@ -281,11 +389,11 @@ int launch_tile_weight_i8(const uint8_t* w, int64_t ldw, int64_t N, int64_t K, u
 
 int launch_quantize_weight(const void* w, int dtype, int64_t N, int64_t K, int64_t ldw, int hblock, int format,
                            void* q, int64_t ldq, void* scale, int64_t ld_scale, void* zero, int64_t ld_zero,
-                           hipStream_t stream) {
+                           int* nonfinite, hipStream_t st) {
     switch (dtype) {
-        case 0: return launch_dt<0>(w, ldw, N, K, hblock, format, q, ldq, scale, ld_scale, zero, ld_zero, stream);
-        case 1: return launch_dt<1>(w, ldw, N, K, hblock, format, q, ldq, scale, ld_scale, zero, ld_zero, stream);
-        case 2: return launch_dt<2>(w, ldw, N, K, hblock, format, q, ldq, scale, ld_scale, zero, ld_zero, stream);
+        case 0: return launch_dt<0>(w, ldw, N, K, hblock, format, q, ldq, scale, ld_scale, zero, ld_zero, nonfinite, st);
+        case 1: return launch_dt<1>(w, ldw, N, K, hblock, format, q, ldq, scale, ld_scale, zero, ld_zero, nonfinite, st);
+        case 2: return launch_dt<2>(w, ldw, N, K, hblock, format, q, ldq, scale, ld_scale, zero, ld_zero, nonfinite, st);
         default: break;
     }
     set_error("quantize_weight: unknown dtype %d", dtype);

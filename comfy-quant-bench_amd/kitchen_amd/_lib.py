@@ -31,6 +31,8 @@ _SIGNATURES = {
                                 c_int),
     "mq_quantize_weight": ([c_vp, c_int, c_i64, c_i64, c_i64, c_int, c_int, c_vp, c_i64, c_vp, c_i64, c_vp, c_i64, c_vp],
                            c_int),
+    "mq_quantize_weight_checked": ([c_vp, c_int, c_i64, c_i64, c_i64, c_int, c_int, c_vp, c_i64, c_vp, c_i64, c_vp,
+                                    c_i64, c_vp, c_vp], c_int),
     "mq_gemm_w4_group": ([c_vp, c_i64, c_vp, c_vp, c_i64, c_vp, c_i64, c_vp, c_i64, c_int, c_int, c_vp, c_int, c_vp,
                           c_int, c_i64, c_i64, c_i64, c_i64, c_vp], c_int),
     "mq_gemm_w4_group_ws": ([c_vp, c_i64, c_vp, c_vp, c_i64, c_vp, c_i64, c_vp, c_i64, c_int, c_int, c_vp, c_int, c_vp,

@@ -160,6 +160,16 @@ int mq_quantize_weight(const void* w, int dtype, int64_t N, int64_t K, int64_t l
                        void* stream);
 
 /*
+ * mq_quantize_weight that also reports a group whose range overflows fp16: *nonfinite (device memory,
+ * or pinned host memory the device can write; NULL: not reported) is set to 1 if any group's scale is
+ * not finite and left as it is otherwise, so the caller clears it before the call and reads it once
+ * the stream has reached the call's end. The row formats never set it.
+ */
+int mq_quantize_weight_checked(const void* w, int dtype, int64_t N, int64_t K, int64_t ldw, int hblock, int format,
+                               void* q, int64_t ldq, void* scale, int64_t ld_scale, void* zero, int64_t ld_zero,
+                               int32_t* nonfinite, void* stream);
+
+/*
  * Load-time decode of comfy-kitchen's shipped asym_w4a8_int8 weight (tools/_formats.py:79-125:
  * qdata I8 [N, K/2] 4-bit codes, s_rel fp8 e4m3fn stored as U8 [N, K/gs], s_channel F32 [N],
  * codebook F32 [16] or none) to an int8 weight with a per-row scale, which the int8 row-scale GEMM

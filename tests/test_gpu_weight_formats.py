@@ -1,0 +1,79 @@
+"""The offline weight quantizer at the edges of its layout (csrc/mq_wquant.hip: 1024-column chunks, four
+waves per row in the row formats), against the oracle, byte for byte."""
+import numpy as np
+import pytest
+import torch
+
+from kitchen_amd import weights
+from oracle import linear, quant
+
+pytestmark = pytest.mark.gpu
+
+
+def _rot(w, cg):
+    return linear.rotate_weight(w, cg) if cg else w
+
+
+# K: one group, groups odd in number, a chunk's end, one past it, four chunks, past four and sixteen
+# (2, 4 and 8 chunks per wave of the row formats); N: a lone row, a ragged last workgroup
+@pytest.mark.parametrize("n,k,cg", [(1, 64, 64), (3, 192, 16), (5, 1024, 256), (7, 1088, 64), (2, 4096, 256),
+                                    (3, 4352, 256), (2, 8256, 64), (1, 16448, 16), (2, 320, 0)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_quantizers(gpu_device, n, k, cg, shift):
+    """shift: the weight starts one element into an odd-strided buffer (element-wise loads)."""
+    print(f"[wquant] N={n} K={k} cg={cg} shift={shift}", flush=True)
+    rng = np.random.default_rng(n * k + cg)
+    w = (rng.standard_normal((n, k)) * 0.02).astype(np.float32)
+    w[:, 5::61] *= 30.0
+    if n > 1:
+        w[1, :64] = 0.0
+    for dtype in (torch.bfloat16, torch.float32):
+        buf = torch.zeros((n, k + 3 * shift), dtype=dtype, device=gpu_device)
+        t = buf[:, shift:shift + k]
+        t.copy_(torch.from_numpy(w).to(dtype))
+        r = _rot(t.float().cpu().numpy(), cg)
+        q, s, z = weights.quantize_w4a8_asym_weight(t, 64, cg)
+        q0, s0, z0 = quant.quant_weight_u4_asym(r, 64)
+        assert np.array_equal(q.cpu().numpy(), quant.pack_u4(q0)) and np.array_equal(z.cpu().numpy(), quant.pack_u4(z0))
+        assert np.array_equal(s.cpu().numpy().view(np.uint16), s0.view(np.uint16))
+        q, s = weights.quantize_w4a4_group_weight(t, 64, cg)
+        q0, s0 = quant.quant_weight_i4_sym_group(r, 64)
+        assert np.array_equal(q.cpu().numpy(), quant.pack_i4(q0))
+        assert np.array_equal(s.cpu().numpy().view(np.uint16), s0.view(np.uint16))
+        q, s = weights.quantize_int8_convrot_weight(t, cg or None)
+        q0, s0 = quant.quant_weight_i8_rowwise(r)
+        assert np.array_equal(q.cpu().numpy(), q0) and np.array_equal(s.cpu().numpy().view(np.uint32), s0.view(np.uint32))
+        if cg:
+            q, s = weights.quantize_convrot_w4a4_weight(t, cg, 64)
+            q0, s0 = quant.quant_weight_i4_rowwise(r)
+            assert np.array_equal(q.cpu().numpy(), quant.pack_i4(q0))
+            assert np.array_equal(s.cpu().numpy().view(np.uint32), s0.view(np.uint32))
+
+
+def test_ties_and_small_scales(gpu_device):
+    """Weights on half-integer multiples of their scale, and groups whose fp16 scale is subnormal."""
+    print("[wquant] ties, subnormal scales", flush=True)
+    rng = np.random.default_rng(5)
+    w = rng.integers(-15, 16, (8, 256)).astype(np.float32) * 0.5
+    w[:, ::64] = 7.0                                  # int4 scale exactly 1 (and 127: int8 ties below)
+    w[4:] *= np.float32(2.0 ** -26)                   # fp16 scales 2^-24 k or 0
+    t = torch.from_numpy(w).to(gpu_device)
+    for fn, ref in ((weights.quantize_w4a4_group_weight, quant.quant_weight_i4_sym_group),
+                    (weights.quantize_w4a8_asym_weight, quant.quant_weight_u4_asym)):
+        got, want = fn(t, 64, 0), ref(w, 64)
+        pack = quant.pack_i4 if fn is weights.quantize_w4a4_group_weight else quant.pack_u4
+        assert np.array_equal(got[0].cpu().numpy(), pack(want[0]))
+        assert np.array_equal(got[1].cpu().numpy().view(np.uint16), want[1].view(np.uint16))
+    w8 = rng.integers(-253, 254, (4, 256)).astype(np.float32) * 0.5
+    w8[:, 0] = 127.0
+    q, s = weights.quantize_int8_convrot_weight(torch.from_numpy(w8).to(gpu_device), None)
+    q0, s0 = quant.quant_weight_i8_rowwise(w8)
+    assert np.array_equal(q.cpu().numpy(), q0) and np.array_equal(s.cpu().numpy(), s0)
+
+
+def test_overflow_is_reported_once_per_call(gpu_device):
+    w = torch.full((4, 2048), 1.0, device=gpu_device)
+    w[3, 2000:] = 3.0e6
+    with pytest.raises(ValueError, match="overflows the fp16 scale"):
+        weights.quantize_w4a4_group_weight(w, 64, 0)
+    weights.quantize_w4a4_group_weight(w[:3], 64, 0)      # the flag is the call's own
