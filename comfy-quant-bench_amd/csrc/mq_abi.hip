@@ -156,6 +156,25 @@ int check_rotquant(const char* what, const void* x, int x_dtype, bool f32_ok, in
     return MQ_OK;
 }
 
+// Argument checks shared by the two codebook decoders (the output's layout is each one's own).
+int check_decode(const void* qdata, int64_t ldq, const void* s_rel, int64_t lds, const float* s_channel,
+                 const float* codebook, int group_size, int64_t N, int64_t K, const int8_t* q8, const float* row_scale) {
+    MQ_REQUIRE(N >= 0 && K > 0, "decode_w4a8_codebook: bad shape N=%lld K=%lld", (long long)N, (long long)K);
+    MQ_REQUIRE(N < (int64_t(1) << 31) && K < (int64_t(1) << 30), "decode_w4a8_codebook: shape too large");
+    MQ_REQUIRE(group_size >= 4 && (16 % group_size == 0 || group_size % 16 == 0),
+               "decode_w4a8_codebook: group_size must be >= 4 and divide or be a multiple of 16 (got %d)", group_size);
+    MQ_REQUIRE(K % 16 == 0 && K % group_size == 0,
+               "decode_w4a8_codebook: K=%lld must be a multiple of 16 and of group_size %d", (long long)K, group_size);
+    if (N == 0) return MQ_OK;
+    MQ_REQUIRE(qdata && s_rel && s_channel && q8 && row_scale, "decode_w4a8_codebook: null pointer");
+    MQ_REQUIRE(ldq >= K / 2 && ldq % 4 == 0 && aligned(qdata, 4),
+               "decode_w4a8_codebook: qdata needs ldq >= K/2 bytes, ldq %% 4 == 0 and a 4-byte aligned base");
+    MQ_REQUIRE(lds >= K / group_size, "decode_w4a8_codebook: s_rel needs lds >= K / group_size bytes");
+    MQ_REQUIRE(aligned(s_channel, 4) && aligned(row_scale, 4) && (!codebook || aligned(codebook, 4)),
+               "decode_w4a8_codebook: fp32 operands must be 4-byte aligned");
+    return MQ_OK;
+}
+
 // The SwiGLU prologue kernels of a mode (MQ_SWIGLU_FUSED / MQ_SWIGLU_EAGER) and input type.
 int launch_swiglu(int mode, int h_dtype, const uint16_t* h, int64_t M, int64_t K, int64_t ldh, int hblock, int bits,
                   int packed, void* q, int64_t ldq, float* scale, hipStream_t st) {
@@ -200,23 +219,29 @@ int mq_decode_w4a8_codebook(const void* qdata, int64_t ldq, const void* s_rel, i
                             const float* codebook, int group_size, int64_t N, int64_t K, int8_t* q8, int64_t ldq8,
                             float* row_scale, void* stream) {
     clear_error();
-    MQ_REQUIRE(N >= 0 && K > 0, "decode_w4a8_codebook: bad shape N=%lld K=%lld", (long long)N, (long long)K);
-    MQ_REQUIRE(N < (int64_t(1) << 31) && K < (int64_t(1) << 30), "decode_w4a8_codebook: shape too large");
-    MQ_REQUIRE(group_size >= 4 && (16 % group_size == 0 || group_size % 16 == 0),
-               "decode_w4a8_codebook: group_size must be >= 4 and divide or be a multiple of 16 (got %d)", group_size);
-    MQ_REQUIRE(K % 16 == 0 && K % group_size == 0,
-               "decode_w4a8_codebook: K=%lld must be a multiple of 16 and of group_size %d", (long long)K, group_size);
-    if (N == 0) return MQ_OK;
-    MQ_REQUIRE(qdata && s_rel && s_channel && q8 && row_scale, "decode_w4a8_codebook: null pointer");
-    MQ_REQUIRE(ldq >= K / 2 && ldq % 4 == 0 && aligned(qdata, 4),
-               "decode_w4a8_codebook: qdata needs ldq >= K/2 bytes, ldq %% 4 == 0 and a 4-byte aligned base");
-    MQ_REQUIRE(lds >= K / group_size, "decode_w4a8_codebook: s_rel needs lds >= K / group_size bytes");
+    const int rc = check_decode(qdata, ldq, s_rel, lds, s_channel, codebook, group_size, N, K, q8, row_scale);
+    if (rc != MQ_OK || N == 0) return rc;
     MQ_REQUIRE(ldq8 >= K && ldq8 % 8 == 0 && aligned(q8, 8),
                "decode_w4a8_codebook: q8 needs ldq8 >= K bytes, ldq8 %% 8 == 0 and an 8-byte aligned base");
-    MQ_REQUIRE(aligned(s_channel, 4) && aligned(row_scale, 4) && (!codebook || aligned(codebook, 4)),
-               "decode_w4a8_codebook: fp32 operands must be 4-byte aligned");
     return launch_decode_w4a8_codebook(static_cast<const uint8_t*>(qdata), ldq, static_cast<const uint8_t*>(s_rel),
-                                       lds, s_channel, codebook, group_size, N, K, q8, ldq8, row_scale,
+                                       lds, s_channel, codebook, group_size, N, K, q8, ldq8, row_scale, false,
+                                       static_cast<hipStream_t>(stream));
+}
+
+int mq_decode_w4a8_codebook_tile16(const void* qdata, int64_t ldq, const void* s_rel, int64_t lds,
+                                   const float* s_channel, const float* codebook, int group_size, int64_t N,
+                                   int64_t K, int8_t* out, float* row_scale, void* stream) {
+    clear_error();
+    const int rc = check_decode(qdata, ldq, s_rel, lds, s_channel, codebook, group_size, N, K, out, row_scale);
+    if (rc != MQ_OK) return rc;
+    MQ_REQUIRE(K >= 192 && K % 64 == 0, "decode_w4a8_codebook_tile16: K=%lld must be a multiple of 64 and >= 192",
+               (long long)K);
+    MQ_REQUIRE((N + 15) / 16 * 16 * K < (int64_t(1) << 31),
+               "decode_w4a8_codebook_tile16: the tiled weight must be under 2 GiB");
+    if (N == 0) return MQ_OK;
+    MQ_REQUIRE(aligned(out, 16), "decode_w4a8_codebook_tile16: out must be 16-byte aligned");
+    return launch_decode_w4a8_codebook(static_cast<const uint8_t*>(qdata), ldq, static_cast<const uint8_t*>(s_rel),
+                                       lds, s_channel, codebook, group_size, N, K, out, 0, row_scale, true,
                                        static_cast<hipStream_t>(stream));
 }
 

@@ -40,10 +40,12 @@ int launch_swiglu_eager_rotquant_bf16(const uint16_t* h, int64_t M, int64_t K, i
 int launch_swiglu_eager_rotquant_f16(const uint16_t* h, int64_t M, int64_t K, int64_t ldh, int hblock, int bits,
                                      int packed, void* q, int64_t ldq, float* scale, hipStream_t stream);
 
-// --- load-time decode of the shipped asym_w4a8_int8 codebook weights (mq_codebook.hip)
+// --- load-time decode of the shipped asym_w4a8_int8 codebook weights (mq_codebook.hip), to rows or
+// (tile) to the 16-row tiles of GemmArgs::wtile
 int launch_decode_w4a8_codebook(const uint8_t* qdata, int64_t ldq, const uint8_t* s_rel, int64_t lds,
                                 const float* s_channel, const float* codebook, int group_size, int64_t N,
-                                int64_t K, int8_t* q8, int64_t ldq8, float* row_scale, hipStream_t stream);
+                                int64_t K, int8_t* q8, int64_t ldq8, float* row_scale, bool tile,
+                                hipStream_t stream);
 
 // --- offline weight quantizer (mq_wquant.hip); dtype / format are MQ_DT_* / MQ_WFMT_*
 int launch_quantize_weight(const void* w, int dtype, int64_t N, int64_t K, int64_t ldw, int hblock, int format,

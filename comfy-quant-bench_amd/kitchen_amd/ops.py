@@ -188,6 +188,12 @@ def decode_w4a8_codebook_weight(qdata: torch.Tensor, s_rel: torch.Tensor, s_chan
     or its U8 bytes [N, K/gs], s_channel F32 [N], codebook F32 [16] or None) to
     (q8 int8 [N, K], row_scale float32 [N]) for the int8 row-scale GEMM; the rule is in
     include/mq.h (mq_decode_w4a8_codebook)."""
+    return _decode_codebook(qdata, s_rel, s_channel, codebook, group_size, False)
+
+
+def _decode_codebook(qdata, s_rel, s_channel, codebook, group_size: int, tiles: bool):
+    """decode_w4a8_codebook_weight, its int8 weight in rows [N, K] or (tiles) in the 16-row tiles of
+    tile_int8_weight."""
     if not qdata.is_cuda:
         raise ValueError("kitchen_amd ops run on the GPU: qdata must be a device tensor")
     q = _u8(qdata)
@@ -203,8 +209,13 @@ def decode_w4a8_codebook_weight(qdata: torch.Tensor, s_rel: torch.Tensor, s_chan
         cb = codebook.reshape(-1).to(device=q.device, dtype=torch.float32).contiguous()
         if cb.numel() != 16:
             raise ValueError(f"codebook must have 16 levels, got {cb.numel()}")
-    q8 = torch.empty((n, k), dtype=torch.int8, device=q.device)
     rs = torch.empty((n,), dtype=torch.float32, device=q.device)
+    if tiles:
+        q8 = torch.empty(((n + 15) // 16, k // 64, 16, 64), dtype=torch.int8, device=q.device)
+        _lib.call("mq_decode_w4a8_codebook_tile16", q.data_ptr(), q.stride(0), sr.data_ptr(), sr.stride(0),
+                  sc.data_ptr(), _lib.ptr(cb), int(group_size), n, k, q8.data_ptr(), rs.data_ptr(), _lib.stream_of(q))
+        return q8, rs
+    q8 = torch.empty((n, k), dtype=torch.int8, device=q.device)
     _lib.call("mq_decode_w4a8_codebook", q.data_ptr(), q.stride(0), sr.data_ptr(), sr.stride(0), sc.data_ptr(),
               _lib.ptr(cb), int(group_size), n, k, q8.data_ptr(), q8.stride(0), rs.data_ptr(), _lib.stream_of(q))
     return q8, rs
@@ -622,10 +633,10 @@ class PreparedW4A8:
     the row-scale GEMM takes; calling it runs only rotate + quantize and the int8 GEMM."""
 
     def __init__(self, qdata, s_rel, s_channel, codebook=None, group_size: int = 16, convrot_groupsize: int = 256):
-        q8, self.row_scale = decode_w4a8_codebook_weight(qdata, s_rel, s_channel, codebook, group_size)
-        self.n, self.k = q8.shape
+        self.n, self.k = qdata.shape[0], qdata.shape[1] * 2
         # held in 16-row tiles where the GEMM takes them (same results, whole-line weight loads)
-        self.q8 = tile_int8_weight(q8) if self.k >= 192 and self.k % 64 == 0 else q8
+        tiles = self.k >= 192 and self.k % 64 == 0
+        self.q8, self.row_scale = _decode_codebook(qdata, s_rel, s_channel, codebook, group_size, tiles)
         self.convrot_groupsize = convrot_groupsize
 
     def __call__(self, x, bias=None, out_dtype=None):

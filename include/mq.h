@@ -197,6 +197,15 @@ int mq_decode_w4a8_codebook(const void* qdata, int64_t ldq, const void* s_rel, i
                             float* row_scale, void* stream);
 
 /*
+ * The same decode straight into the 16-row tiles of MQ_W8_TILE16 (mq_tile_weight_i8 of the rows, in one
+ * pass): out [ceil(N/16)][K/64][16][64] int8, 16-byte aligned, rows past N zero. Needs K % 64 == 0,
+ * K >= 192 and tiles under 2 GiB.
+ */
+int mq_decode_w4a8_codebook_tile16(const void* qdata, int64_t ldq, const void* s_rel, int64_t lds,
+                                   const float* s_channel, const float* codebook, int group_size, int64_t N,
+                                   int64_t K, int8_t* out, float* row_scale, void* stream);
+
+/*
  * Load-time expansion of packed 4-bit weights [N, K/2] (uint4 with zero-points wz, or signed int4
  * when wz is NULL) to int8 in the 16-row tiles of MQ_W8_TILE16, [ceil(N/16)][K/64][16][64] bytes
  * (rows past N zero). Byte (n, k) is v = q - z[n, k/64] (uint4) or the signed nibble, then by

@@ -1,10 +1,13 @@
-"""The offline weight quantizer at the edges of its layout (csrc/mq_wquant.hip: 1024-column chunks, four
-waves per row in the row formats), against the oracle, byte for byte."""
+"""The offline weight quantizer and the codebook decoder at the edges of their layouts (csrc/mq_wquant.hip:
+1024-column chunks, four waves per row in the row formats; csrc/mq_codebook.hip: 16-row tiles), against
+the oracle, byte for byte."""
 import numpy as np
 import pytest
 import torch
 
-from kitchen_amd import weights
+import kitchen_amd as ck
+from kitchen_amd import _lib, ops, weights
+from oracle import codebook as cbk
 from oracle import linear, quant
 
 pytestmark = pytest.mark.gpu
@@ -77,3 +80,30 @@ def test_overflow_is_reported_once_per_call(gpu_device):
     with pytest.raises(ValueError, match="overflows the fp16 scale"):
         weights.quantize_w4a4_group_weight(w, 64, 0)
     weights.quantize_w4a4_group_weight(w[:3], 64, 0)      # the flag is the call's own
+
+
+@pytest.mark.parametrize("n,k,gs", [(1, 192, 4), (16, 256, 8), (17, 1024, 16), (40, 1088, 32), (33, 3072, 64), (5, 192, 192)])
+@pytest.mark.parametrize("shift", [0, 4])
+def test_decode_to_tiles(gpu_device, n, k, gs, shift):
+    """PreparedW4A8's tiles: the decoded rows, tiled; shift: packed rows aligned to 4 bytes only."""
+    print(f"[codebook] tiles N={n} K={k} gs={gs} shift={shift}", flush=True)
+    rng = np.random.default_rng(n + k + gs)
+    qd = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
+    sr = rng.integers(0, 256, (n, k // gs), dtype=np.uint8)            # every fp8 byte, NaN included
+    sc = rng.uniform(0.001, 0.05, n).astype(np.float32)
+    cb = np.sort(rng.uniform(-1, 1, 16)).astype(np.float32)
+    buf = torch.zeros((n, k // 2 + shift), dtype=torch.uint8, device=gpu_device)
+    q = buf[:, shift:] if shift else buf
+    q.copy_(torch.from_numpy(qd))
+    q0, _ = cbk.decode_w4a8_codebook(qd, sr, sc, cb, gs)
+    args = (torch.from_numpy(sr).to(gpu_device), torch.from_numpy(sc).to(gpu_device), torch.from_numpy(cb).to(gpu_device))
+    rows, rs = torch.empty((n, k), dtype=torch.int8, device=gpu_device), torch.empty(n, device=gpu_device)
+    tiles = torch.full(((n + 15) // 16, k // 64, 16, 64), 99, dtype=torch.int8, device=gpu_device)
+    head = (q.data_ptr(), q.stride(0), args[0].data_ptr(), k // gs, args[1].data_ptr(), args[2].data_ptr(), gs, n, k)
+    _lib.call("mq_decode_w4a8_codebook", *head, rows.data_ptr(), k, rs.data_ptr(), _lib.stream_of(q))
+    assert np.array_equal(rows.cpu().numpy(), q0) and np.array_equal(rs.cpu().numpy(), sc)
+    rs.zero_()
+    _lib.call("mq_decode_w4a8_codebook_tile16", *head, tiles.data_ptr(), rs.data_ptr(), _lib.stream_of(q))
+    assert torch.equal(tiles, ops.tile_int8_weight(rows)) and np.array_equal(rs.cpu().numpy(), sc)
+    p = ck.PreparedW4A8(q, *args, gs)
+    assert (p.n, p.k) == (n, k) and torch.equal(p.q8, tiles) and torch.equal(p.row_scale, rs)
