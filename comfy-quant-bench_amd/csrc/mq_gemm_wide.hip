@@ -65,17 +65,16 @@ typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 constexpr int TK = 64;
 constexpr int LAG = 3;                    // tile t's fmas run LAG MFMAs after it
 constexpr int kSeed = 0x4B400000;         // bits of 1.5 * 2^23
-constexpr int NSTAGE = 4;
 
-// Tile configuration and LDS map (bytes): 4-stage rings of A tiles, unpacked B tiles and fp32
+// Tile configuration and LDS map (bytes): NSTAGE-stage (4, or 8) rings of A tiles, unpacked B tiles and fp32
 // scales; the output staging of the epilogue reuses the ring region. The B stages have TM rows like
 // the A stages, so every thread keeps the same load and store roles; rows TN .. TM - 1 of a B stage
 // (256 x 192 tile) receive only zeros and are never read. 256 tiles: A / B stages of 16 KB, 137 KB
 // in all; 128 tile: 8 KB stages, 67.5 KB in all.
 constexpr int NT = 512;                                       // threads per workgroup: 8 waves
-template <int TM_, int TN_>
+template <int TM_, int TN_, int NS_ = 4>
 struct Cfg {
-    static constexpr int TM = TM_, TN = TN_;
+    static constexpr int TM = TM_, TN = TN_, NSTAGE = NS_;
     static constexpr int WR = TM / 4, WC = TN / 2;            // wave tile (4 x 2 waves)
     static constexpr int NI = WR / 16, NJ = WC / 16;          // MFMA row / column tiles per wave
     static constexpr int NTL = NI * NJ;                       // MFMA tiles per wave and K group
@@ -95,7 +94,7 @@ struct Cfg {
     static constexpr int SMEM_BYTES = BI_LDS + TN * 4;
 };
 static_assert(Cfg<256, 256>::SMEM_BYTES <= 160 * 1024 && Cfg<256, 192>::SMEM_BYTES <= 160 * 1024 &&
-                  Cfg<128, 128>::SMEM_BYTES <= 160 * 1024, "LDS budget");
+                  Cfg<128, 128>::SMEM_BYTES <= 160 * 1024 && Cfg<128, 128, 8>::SMEM_BYTES <= 160 * 1024, "LDS budget");
 
 // LDS operations a wave issues in a group after its last LDS store (step ts): the B fragment reads
 // (steps with i == 0), the next group's A fragment reads and, with group scales, the scale reads
@@ -274,9 +273,19 @@ __device__ __forceinline__ T& lds(uint8_t* smem, int off) {
 // expanded to int8 in 16-row tiles (mq_expand_weight_w4: the bytes the unpack would store, zero-point
 // and sign included), so B takes A's DMA path and no zero-points are loaded; the arithmetic, and
 // the scaling by WK and AM, is the packed kernel's.
-template <int TM_, int TN_, WKind WK, Epi EPI, int AM, bool SPLIT, bool XP>
+//
+// NS: stages of the LDS ring. Eight for the 128 x 128 tile's int8 row-scale products when every compute
+// unit has at most one workgroup: their groups are short (eight MFMAs per wave and nothing else), so
+// four stages give the DMA of a group, two groups' time to arrive, less than its latency. W8A8 linears,
+// us, 4 -> 8 stages: 256 x 3072 x 3072 18.9 -> 16.5, 200 x 4000 x 3072 18.7 -> 16.6, 256 x 12288 x 3072
+// 21.0 -> 19.8, 1024 x 3072 x 3072 23.6 -> 22.6. The group-scale products, bound by the VALU and LDS work
+// of their groups, gain nothing (1024 x 3072 x 3072 30.3 -> 31.0) and keep four; so do larger launches,
+// which fit two such workgroups' LDS on a compute unit.
+template <int TM_, int TN_, WKind WK, Epi EPI, int AM, bool SPLIT, bool XP, int NS>
 __global__ void __launch_bounds__(NT) gemm_wide_kernel(GemmArgs a, int tiles_m, int tiles_n) {
-    using C = Cfg<TM_, TN_>;
+    using C = Cfg<TM_, TN_, NS>;
+    static_assert(NS == 4 || (NS == 8 && TM_ == 128 && WK == WKind::I8 && EPI == Epi::RowScale), "stages");
+    constexpr int kAhead = NS - 1;   // K groups the DMA runs ahead
     constexpr int TM = C::TM, TN = C::TN, NI = C::NI, NJ = C::NJ, NTL = C::NTL, TILE_BYTES = C::TILE_BYTES;
     constexpr int WR = C::WR, WC = C::WC, NH = C::NH, TPR = C::TPR;
     constexpr int A_LDS = C::A_LDS, B_LDS = C::B_LDS, S_LDS = C::S_LDS, OROW = C::OROW;
@@ -635,18 +644,29 @@ __global__ void __launch_bounds__(NT) gemm_wide_kernel(GemmArgs a, int tiles_m, 
     store_b(1, 1, I1{}, I1{}, 0);
     store_b(1, 1, I1{}, I1{}, 1);
     store_s(1, g0 + 1, I1{}, I1{});
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // A(0), A(1) of every kind (int8 B has no B loads)
+    constexpr int kDmaOps = NH * (kPacked ? 1 : 2);   // VMEM operations of a group's DMA per thread
+    if constexpr (NS == 8) {
+        // A(2) .. A(6) and their B go out before the wait for A(0) and A(1), which leaves them in flight
+#pragma unroll
+        for (int u = 2; u < kAhead; ++u) dma_group(g0 + u, u);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kAhead - 2) * kDmaOps) : "memory");
+    } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // A(0), A(1) of every kind (int8 B has no B loads)
+    }
+    // (inline-asm stores: an ordinary LDS store would wait for the DMA in flight)
     if constexpr (kFinal) {
         if (tid < TM) {
-            lds<float>(smem, R_LDS + 4 * tid) = ep_a;
+            ds_write4<4>(R_LDS + 4 * tid, 0, ep_a);
         } else if (tid - TM < TN) {
-            lds<float>(smem, BI_LDS + 4 * (tid - TM)) = ep_a;
-            if constexpr (EPI == Epi::RowScale) lds<float>(smem, C_LDS + 4 * (tid - TM)) = ep_b;
+            ds_write4<4>(BI_LDS + 4 * (tid - TM), 0, ep_a);
+            if constexpr (EPI == Epi::RowScale) ds_write4<4>(C_LDS + 4 * (tid - TM), 0, ep_b);
         }
     }
-    gload_b(g0 + 2, 0);
-    dma_group(g0 + 2, 2);
-    gload_b(g0 + 3, 1);
+    if constexpr (NS == 4) {
+        gload_b(g0 + 2, 0);
+        dma_group(g0 + 2, 2);
+        gload_b(g0 + 3, 1);
+    }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -667,7 +687,6 @@ __global__ void __launch_bounds__(NT) gemm_wide_kernel(GemmArgs a, int tiles_m, 
     // kXS: group g + 1's scales load at step LAG of group g (once group g - 1's last fmas, steps
     // 0 .. LAG - 1, have read that slot), ahead of the group's DMA; the wait before the barrier that
     // ends group g takes them (kTD > LAG).
-    constexpr int kDmaOps = NH * (kPacked ? 1 : 2);
     constexpr int kTD = kPacked ? 0 : kXS && 8 % NTL <= LAG ? LAG + 1 : 8 % NTL;
     static_assert(!kXS || kTD > LAG, "the scales load before the group's DMA");
     // steps of the B unpack (kTB: wait for the registers, store; kTB + 1: second half for T = 256),
@@ -698,10 +717,15 @@ __global__ void __launch_bounds__(NT) gemm_wide_kernel(GemmArgs a, int tiles_m, 
         EPI == Epi::GroupPartials ? 0 : kXS ? 1 + kDmaOps : (kZS > 0 ? kDmaOps : 2 * kDmaOps + kB),
         EPI == Epi::GroupPartials ? 0 : kXS ? 63 : 2 * kDmaOps + kB + kZS};
 
-    // K group g with A stage, B stage and register set fixed by U = g % 4 (compile-time). Step t = NI j + i.
+    // Eight stages: before the barrier that ends group g, A(g + 2) (issued in group g - 5) must be
+    // complete; issued after it: the DMA of groups g - 4 .. g.
+    constexpr int kDeepAfter = (kAhead - 2) * kDmaOps;
+
+    // K group g with A stage, B stage and register set fixed by U = g % NS (compile-time). Step t = NI j + i.
     auto group = [&](int g, auto Uc) {
         constexpr int U = decltype(Uc)::value;
-        constexpr int ST = U, ST1 = (U + 1) % 4, ST2 = (U + 2) % 4, ST3 = (U + 3) % 4, SET = U % 2;
+        constexpr int ST = U, ST1 = (U + 1) % NS, ST2 = (U + 2) % NS, STA = (U + kAhead) % NS, SET = U % 2;
+        constexpr int U4 = U % 4;                                // position in the block of four
         using PARc = std::integral_constant<int, U % 2>;
         using U2c = std::integral_constant<int, (U + 2) % 4>;   // position of group g + 2 in its block
         constexpr int PAR = PARc::value;
@@ -724,7 +748,7 @@ __global__ void __launch_bounds__(NT) gemm_wide_kernel(GemmArgs a, int tiles_m, 
             }
             if constexpr (kXS)
                 if (t == LAG) gload_sc(g + 1, PAR ^ 1);
-            if (t == kTD) dma_group(g + 3, ST3);
+            if (t == kTD) dma_group(g + kAhead, STA);
             // B fragments three columns ahead (the next group's first columns from stage ST1,
             // complete since the barrier that ended group g - 1)
             if (i == 0) {
@@ -745,9 +769,9 @@ __global__ void __launch_bounds__(NT) gemm_wide_kernel(GemmArgs a, int tiles_m, 
             if (i == (NI == 4 ? 2 : 1) && j < NI) read_a(ST1, SET ^ 1, j);
             // unpack register set SET (group g + 2, parity PAR) into stage ST2, then reload it with g + 4
             if (t == kTB) {
-                MQ_WAIT_B(kWaitB[U], SET);
+                if constexpr (NS == 4) MQ_WAIT_B(kWaitB[U4], SET);
                 // group g + 2 opens the block of zero-points and scales loaded in group g - 1
-                if constexpr (U == 2) settle_zs();
+                if constexpr (U4 == 2) settle_zs();
                 store_b(ST2, SET, PARc{}, U2c{}, 0);
             }
             if constexpr (TPR == 2)
@@ -755,7 +779,7 @@ __global__ void __launch_bounds__(NT) gemm_wide_kernel(GemmArgs a, int tiles_m, 
             if (t == kTS) store_s(ST2, g + 2, PARc{}, U2c{});
             if (t == kTL) {
                 gload_b(g + 4, SET);
-                if constexpr (U == 1) gload_zs(g + 3);
+                if constexpr (U4 == 1) gload_zs(g + 3);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -767,10 +791,10 @@ __global__ void __launch_bounds__(NT) gemm_wide_kernel(GemmArgs a, int tiles_m, 
         // (the next group's fragment and scale reads, which stay in flight across the barrier).
         // Group g's own stages were last read by MFMAs that have issued.
         // (kXS: group g + 1's scales, slot PAR ^ 1, arrive with the same wait. kXS stores nothing to LDS
-        // in the loop, so no LDS wait is needed.)
-        if constexpr (kXS) wait_sc(std::integral_constant<int, kVmAfter[U]>{}, std::integral_constant<int, PAR ^ 1>{});
-        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kVmAfter[U]) : "memory");
-        if constexpr (NJ != 8 && !kXS) {
+        // in the loop, so no LDS wait is needed; nor do int8 weights with row scales.)
+        if constexpr (kXS) wait_sc(std::integral_constant<int, kVmAfter[U4]>{}, std::integral_constant<int, PAR ^ 1>{});
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NS == 8 ? kDeepAfter : kVmAfter[U4]) : "memory");
+        if constexpr (NJ != 8 && !kXS && (kPacked || EPI == Epi::GroupScale)) {
             constexpr int kLdsAfter = lds_ops_after(NI, NJ, kTS, EPI == Epi::GroupScale);
             static_assert(kLdsAfter < 16, "lgkmcnt holds 0-15");
             asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(kLdsAfter) : "memory");
@@ -779,11 +803,17 @@ __global__ void __launch_bounds__(NT) gemm_wide_kernel(GemmArgs a, int tiles_m, 
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
-    for (int g = g0; g < g1; g += 4) {
+    for (int g = g0; g < g1; g += NS) {
         group(g, std::integral_constant<int, 0>{});
         group(g + 1, std::integral_constant<int, 1>{});
         group(g + 2, std::integral_constant<int, 2>{});
         group(g + 3, std::integral_constant<int, 3>{});
+        if constexpr (NS == 8) {
+            group(g + 4, std::integral_constant<int, 4>{});
+            group(g + 5, std::integral_constant<int, 5>{});
+            group(g + 6, std::integral_constant<int, 6>{});
+            group(g + 7, std::integral_constant<int, 7>{});
+        }
     }
     // The last K groups issued loads for groups past the end (zero-size resources) that nothing
     // waits for: B registers, zero-points, scales and stage DMA. Their data may land at any time
@@ -1017,13 +1047,11 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(GemmArgs a) {
     }
 }
 
-template <int TM, int TN, WKind WK, Epi EPI, int AM, bool XP>
-int launch_tile(const GemmArgs& a, hipStream_t stream) {
-    const int tiles_m = static_cast<int>((a.M + TM - 1) / TM);
-    const int tiles_n = static_cast<int>((a.N + TN - 1) / TN);
+template <int TM, int TN, WKind WK, Epi EPI, int AM, bool XP, int NS>
+int launch_ring(const GemmArgs& a, int tiles_m, int tiles_n, hipStream_t stream) {
     if constexpr (EPI == Epi::GroupScale || EPI == Epi::RowScale) {
         if (a.ksplit > 1) {
-            hipLaunchKernelGGL((gemm_wide_kernel<TM, TN, WK, EPI, AM, true, XP>),
+            hipLaunchKernelGGL((gemm_wide_kernel<TM, TN, WK, EPI, AM, true, XP, NS>),
                                dim3(static_cast<unsigned>(tiles_m * tiles_n * a.ksplit)), dim3(NT), 0, stream, a,
                                tiles_m, tiles_n);
             const int rc = launch_status("gemm_wide");
@@ -1034,9 +1062,22 @@ int launch_tile(const GemmArgs& a, hipStream_t stream) {
             return launch_status("gemm_splitk_reduce");
         }
     }
-    hipLaunchKernelGGL((gemm_wide_kernel<TM, TN, WK, EPI, AM, false, XP>), dim3(static_cast<unsigned>(tiles_m * tiles_n)),
+    hipLaunchKernelGGL((gemm_wide_kernel<TM, TN, WK, EPI, AM, false, XP, NS>), dim3(static_cast<unsigned>(tiles_m * tiles_n)),
                        dim3(NT), 0, stream, a, tiles_m, tiles_n);
     return launch_status("gemm_wide");
+}
+
+template <int TM, int TN, WKind WK, Epi EPI, int AM, bool XP>
+int launch_tile(const GemmArgs& a, hipStream_t stream) {
+    const int tiles_m = static_cast<int>((a.M + TM - 1) / TM);
+    const int tiles_n = static_cast<int>((a.N + TN - 1) / TN);
+    // eight stages (see the kernel) where the K groups of every workgroup make whole rounds of that ring:
+    // an exit in mid-round would cost the accumulators' moves on every round
+    if constexpr (TM == 128 && WK == WKind::I8 && EPI == Epi::RowScale)
+        if (static_cast<int64_t>(tiles_m) * tiles_n * a.ksplit <= device_cu_count() && (a.K / TK + 3) / 4 % 2 == 0 &&
+            a.kgroups % 8 == 0)
+            return launch_ring<TM, TN, WK, EPI, AM, XP, 8>(a, tiles_m, tiles_n, stream);
+    return launch_ring<TM, TN, WK, EPI, AM, XP, 4>(a, tiles_m, tiles_n, stream);
 }
 
 template <WKind WK, Epi EPI, int AM, bool XP = false>
