@@ -1,6 +1,7 @@
-"""Build libmq.so (the gfx950 HIP kernels + C ABI) in-tree with hipcc.
+"""Build libmq.so (the gfx950 HIP kernels + C ABI) in-tree with hipcc, and the CPython module that calls
+its per-call entry points (csrc/mq_fast.c) with the C compiler.
 
-    python comfy-quant-bench_amd/build.py            # -> comfy-quant-bench_amd/kitchen_amd/libmq.so
+    python comfy-quant-bench_amd/build.py            # -> comfy-quant-bench_amd/kitchen_amd/libmq.so, _fast.so
 
 The library is written for gfx950 only. Every HIP source is compiled with packed fp32
 instructions disabled (target feature -packed-fp32-ops) and with floating-point contraction off:
@@ -14,10 +15,12 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "kitchen_amd", "libmq.so")
+FAST = os.path.join(HERE, "kitchen_amd", "_fast.so")
 SOURCES = ["mq_abi.hip", "mq_rotquant.hip", "mq_rotquant_f16.hip", "mq_rotquant_f32.hip", "mq_swiglu.hip",
            "mq_swiglu_f16.hip", "mq_swiglu_eager.hip", "mq_swiglu_eager_f16.hip",
            "mq_codebook.hip", "mq_wquant.hip", "mq_gemv.hip", "mq_gemm.hip", "mq_gemm_few.hip",
@@ -63,6 +66,17 @@ def _compile(src: str, build_dir: str, verbose: bool) -> str:
     return obj
 
 
+def _compile_fast() -> None:
+    cc = shutil.which("gcc") or shutil.which("cc") or os.path.join(os.path.dirname(hipcc()), "amdclang")
+    tmp = FAST + ".tmp"
+    cmd = [cc, "-O2", "-shared", "-fPIC", "-Wall", "-Wno-unused-function", "-I", sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "mq_fast.c"), "-o", tmp]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{cc} failed on mq_fast.c:\n{res.stderr}")
+    os.replace(tmp, FAST)
+
+
 def build(verbose: bool = False) -> str:
     """Compile every source (in parallel) and link libmq.so; returns its path. Always recompiles."""
     build_dir = os.path.join(HERE, "_build")
@@ -71,6 +85,7 @@ def build(verbose: bool = False) -> str:
     subprocess.run([sys.executable, os.path.join(CSRC, "gen_silu_table.py"),
                     os.path.join(build_dir, "gen", "mq_silu_table.h"),
                     os.path.join(build_dir, "gen", "mq_silu_f16_table.h")], check=True)
+    _compile_fast()
     workers = max(1, min(len(SOURCES), os.cpu_count() or 1))
     with concurrent.futures.ThreadPoolExecutor(max_workers=workers) as pool:
         objs = list(pool.map(lambda src: _compile(src, build_dir, verbose), SOURCES))

@@ -1,5 +1,8 @@
 """ctypes binding of libmq.so (C ABI in include/mq.h).
 
+The entry points that a linear or an activation quantizer makes per call go through the CPython module
+_fast.so (csrc/mq_fast.c), bound to the same loaded library; all others through ctypes.
+
 The library is loaded after `import torch`, so its `libamdhip64.so.7` dependency resolves to the
 HIP runtime torch already mapped: device pointers, streams and the kernels share one runtime.
 There is no fallback: if the library is missing, every call raises.
@@ -16,6 +19,8 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmq.so")
 
 _lib = None
+FAST_ENTRIES = ("mq_rotquant", "mq_swiglu_rotquant", "mq_linear_w4_group", "mq_linear_rowscale")
+_entries: dict = {}   # entry point name -> callable
 
 c_i64 = ctypes.c_int64
 c_int = ctypes.c_int
@@ -101,15 +106,24 @@ def load() -> ctypes.CDLL:
     ver = lib.mq_abi_version()
     if ver != ABI_VERSION:
         raise RuntimeError(f"libmq ABI version {ver}, expected {ABI_VERSION}: rebuild the library")
+    try:
+        from . import _fast
+    except ImportError as e:
+        raise RuntimeError(f"{os.path.join(_HERE, '_fast.so')} is not built: run `python comfy-quant-bench_amd/build.py` "
+                           "(or __graft_entry__.build()) first") from e
+    _fast.bind(*(ctypes.cast(getattr(lib, name), c_vp).value for name in FAST_ENTRIES))
+    _entries.update({name: getattr(lib, name) for name in _SIGNATURES})
+    _entries.update({name: getattr(_fast, name) for name in FAST_ENTRIES})
     _lib = lib
     return lib
 
 
 def call(name: str, *args) -> None:
-    lib = load()
-    rc = getattr(lib, name)(*args)
+    if _lib is None:
+        load()
+    rc = _entries[name](*args)
     if rc != 0:
-        msg = lib.mq_last_error().decode(errors="replace")
+        msg = _lib.mq_last_error().decode(errors="replace")
         if rc == -1:
             raise ValueError(f"{name}: {msg}")
         raise MQError(f"{name} failed ({rc}): {msg}")

@@ -52,8 +52,9 @@ def _as_2d(x: torch.Tensor, k: int) -> torch.Tensor:
         raise ValueError("kitchen_amd ops run on the GPU: x must be a device tensor")
     if x.dtype not in FLOAT_TYPES:
         raise ValueError(f"x must be bfloat16, float16 or float32, got {x.dtype}")
-    # a contiguous 2-D x is what the reshape would return: used as it is (no new view per call)
-    if x.dim() == 2 and x.shape[1] == k and x.stride(1) == 1 and x.stride(0) == k:
+    # a contiguous 2-D x is what the reshape would return: used as it is (no new view per call); its
+    # rows are k elements apart, whatever the stride of a single row says
+    if x.dim() == 2 and x.shape[1] == k and x.is_contiguous():
         return x
     return x.reshape(-1, k).contiguous()
 
@@ -235,15 +236,18 @@ def _check_w4_group_weights(qweight, wscales, wzeros, n, k, group_size):
     if qweight is not None and (qweight.shape != (n, k // 2) or qweight.element_size() != 1):
         raise ValueError(f"qweight must be 8-bit [{n}, {k // 2}]")
     groups = k // group_size
-    if wscales is not None and (wscales.dtype != torch.float16 or wscales.shape[0] != n
-                                or wscales.shape[1] < groups or wscales.stride(1) != 1):
-        raise ValueError(f"wscales must be float16 [{n}, {groups}] with unit column stride")
-    if wzeros is not None and (wzeros.element_size() != 1 or wzeros.shape[0] != n
-                               or wzeros.shape[1] < (groups + 1) // 2 or wzeros.stride(1) != 1):
-        raise ValueError(f"zero-points must be packed uint4 [{n}, {(groups + 1) // 2}]")
+    if wscales is not None:
+        shape = wscales.shape
+        if wscales.dtype != torch.float16 or shape[0] != n or shape[1] < groups or wscales.stride(1) != 1:
+            raise ValueError(f"wscales must be float16 [{n}, {groups}] with unit column stride")
+    if wzeros is not None:
+        shape = wzeros.shape
+        if wzeros.element_size() != 1 or shape[0] != n or shape[1] < (groups + 1) // 2 or wzeros.stride(1) != 1:
+            raise ValueError(f"zero-points must be packed uint4 [{n}, {(groups + 1) // 2}]")
 
 
 _WS_BYTES: dict = {}
+_LINEAR_WS_BYTES: dict = {}
 
 # Workspaces up to this size are kept per (device, stream) and reused by the next call on that
 # stream (calls on one stream run in order, so they never overlap); larger ones, and every
@@ -253,10 +257,10 @@ WORKSPACE_CACHE_BYTES = 64 << 20
 _WS_CACHE: dict = {}
 
 
-def _scratch(nbytes: int, device) -> torch.Tensor:
+def _scratch(nbytes: int, device, stream: int) -> torch.Tensor:
     if nbytes > WORKSPACE_CACHE_BYTES or torch.cuda.is_current_stream_capturing():
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
-    key = (device.index, _lib.stream_of_device(device))
+    key = (device.index, stream)
     buf = _WS_CACHE.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = _WS_CACHE[key] = torch.empty(nbytes, dtype=torch.uint8, device=device)
@@ -271,18 +275,18 @@ def _workspace(m: int, n: int, k: int, device):
     if nbytes is None:
         with torch.cuda.device(device):
             nbytes = _WS_BYTES[key] = int(_lib.load().mq_gemm_workspace_bytes(m, n, k))
-    return _scratch(nbytes, device) if nbytes > 0 else None
+    return _scratch(nbytes, device, _lib.stream_of_device(device)) if nbytes > 0 else None
 
 
-def _linear_workspace(m: int, n: int, k: int, device) -> torch.Tensor:
-    """Workspace of the whole-linear entry points (activation codes, scales and split-K partials),
-    its size asked of the library once per shape and device."""
-    key = ("linear", device.index, m, n, k)
-    nbytes = _WS_BYTES.get(key)
+def _linear_workspace(m: int, n: int, k: int, device, stream: int) -> torch.Tensor:
+    """Workspace of the whole-linear entry points (activation codes, scales and split-K partials) for a
+    call on `stream`, its size asked of the library once per shape and device."""
+    key = (device.index, m, n, k)
+    nbytes = _LINEAR_WS_BYTES.get(key)
     if nbytes is None:
         with torch.cuda.device(device):
-            nbytes = _WS_BYTES[key] = int(_lib.load().mq_linear_workspace_bytes(m, n, k))
-    return _scratch(nbytes, device)
+            nbytes = _LINEAR_WS_BYTES[key] = int(_lib.load().mq_linear_workspace_bytes(m, n, k))
+    return _scratch(nbytes, device, stream)
 
 
 def _bias_args(bias):
@@ -539,11 +543,16 @@ def convrot_w4a4_linear(x: torch.Tensor, qweight: torch.Tensor, wscales: torch.T
         ws = wscales.to(torch.float16).contiguous()
         y = _linear_w4_group(x, swiglu, convrot_groupsize, bits, qweight, ws, None, bias, n, k, out_dtype)
     else:
-        ws = wscales.reshape(-1).to(torch.float32).contiguous()
+        ws = _row_scales(wscales)
         if ws.numel() != n:
             raise ValueError(f"per-row wscales must have {n} elements, got {ws.numel()}")
         y = _linear_rowscale(x, swiglu, convrot_groupsize, bits, qweight, 4, ws, bias, n, k, out_dtype)
     return _finish(y, x_out, n)
+
+
+def _row_scales(s: torch.Tensor) -> torch.Tensor:
+    """The per-row weight scales as contiguous fp32 (the tensor itself, of whatever shape, if it is)."""
+    return s if s.dtype == torch.float32 and s.is_contiguous() else s.reshape(-1).to(torch.float32).contiguous()
 
 
 def _linear_input(x: torch.Tensor, swiglu: int, k: int):
@@ -560,24 +569,29 @@ def _linear_w4_group(x, swiglu, cg, act_bits, qweight, wscales, wzeros, bias, n,
     x2, swiglu = _linear_input(x, swiglu, k)
     m = x2.shape[0]
     _check_w4_group_weights(qweight, wscales, wzeros, n, k, INT4_GROUP_SIZE)
-    b = _bias(bias, n, x2.device)
-    y = torch.empty((m, n), dtype=out_dtype, device=x2.device)
+    dev = x2.device
+    b = _bias(bias, n, dev)
+    y = x2.new_empty((m, n)) if out_dtype is x2.dtype else x2.new_empty((m, n), dtype=out_dtype)
     if m == 0:
         return y
-    work = _linear_workspace(m, n, k, x2.device)
-    xw = _expansion(qweight, wzeros, _lib.ACT_X16ALT if act_bits == 4 else _lib.ACT_I8, m, k, wscales)
+    stream = _lib.stream_of_device(dev)
+    work = _linear_workspace(m, n, k, dev, stream)
+    xw = None if m <= FEW_ROWS else \
+        _expansion(qweight, wzeros, _lib.ACT_X16ALT if act_bits == 4 else _lib.ACT_I8, m, k, wscales)
     if xw is not None:
-        qptr, ldw, ab = xw.tiles.data_ptr(), k, int(act_bits) | _lib.W4_EXPANDED
+        qptr, ldw, ab = xw.tiles.data_ptr(), k, act_bits | _lib.W4_EXPANDED
         zptr, ldwz = (xw.tiles.data_ptr() if xw.asym else None), 0   # non-null: uint4 (not read)
     else:
         qw = qweight.contiguous()
-        zz = None if wzeros is None else wzeros.contiguous()
-        qptr, ldw, ab = qw.data_ptr(), qw.stride(0), int(act_bits)
-        zptr, ldwz = _lib.ptr(zz), (0 if zz is None else zz.stride(0))
-    _lib.call("mq_linear_w4_group", x2.data_ptr(), _lib.dtype_code(x2.dtype), x2.stride(0), int(cg or 0), ab,
-              int(swiglu), qptr, ldw, wscales.data_ptr(), wscales.stride(0), zptr, ldwz, *_bias_args(b),
-              y.data_ptr(), _lib.dtype_code(out_dtype), y.stride(0), m, n, k, work.data_ptr(), work.numel(),
-              _lib.stream_of(x2))
+        qptr, ldw, ab = qw.data_ptr(), k // 2, act_bits
+        zptr, ldwz = None, 0
+        if wzeros is not None:
+            zz = wzeros.contiguous()
+            zptr, ldwz = zz.data_ptr(), zz.shape[1]
+    bptr, bdt = (None, _lib.DT_BF16) if b is None else (b.data_ptr(), _lib.DTYPE_CODE[b.dtype])
+    _lib.call("mq_linear_w4_group", x2.data_ptr(), _lib.DTYPE_CODE[x2.dtype], 2 * k if swiglu else k, cg or 0, ab,
+              swiglu, qptr, ldw, wscales.data_ptr(), wscales.stride(0), zptr, ldwz, bptr, bdt, y.data_ptr(),
+              _lib.DTYPE_CODE[out_dtype], n, m, n, k, work.data_ptr(), work.numel(), stream)
     return y
 
 
@@ -585,25 +599,28 @@ def _linear_rowscale(x, swiglu, cg, act_bits, qweight, wbits, wscales, bias, n, 
     """rotate + quantize + row-scale GEMM in one library call (mq_linear_rowscale)."""
     x2, swiglu = _linear_input(x, swiglu, k)
     m = x2.shape[0]
-    qw = qweight if is_tile16(qweight) else qweight.contiguous()
+    tiles = is_tile16(qweight)
+    qw = qweight if tiles else qweight.contiguous()
     wbytes = k // 2 if wbits == 4 else k
-    if not is_tile16(qw) and (qw.shape != (n, wbytes) or qw.element_size() != 1):
+    if not tiles and (qw.shape != (n, wbytes) or qw.element_size() != 1):
         raise ValueError(f"weight must be 8-bit [{n}, {wbytes}]")
-    if wbits == 4:
+    if wbits == 4 and m > GEMV_ROWS:
         # signed int4 rows: their int8 expansion where the wide kernel reads it (same int32 sums)
         xw = _expansion(qweight, None, _lib.W4X_ROW, m, k)
         if xw is not None:
-            qw, wbits = xw.tiles, 8
-    ldw, wbits = _weight_args(qw, n, k, int(wbits))
-    b = _bias(bias, n, x2.device)
-    y = torch.empty((m, n), dtype=out_dtype, device=x2.device)
+            qw, wbits, tiles = xw.tiles, 8, True
+    ldw, wbits = _weight_args(qw, n, k, wbits) if tiles else (wbytes, wbits)
+    dev = x2.device
+    b = _bias(bias, n, dev)
+    y = x2.new_empty((m, n)) if out_dtype is x2.dtype else x2.new_empty((m, n), dtype=out_dtype)
     if m == 0:
         return y
-    work = _linear_workspace(m, n, k, x2.device)
-    _lib.call("mq_linear_rowscale", x2.data_ptr(), _lib.dtype_code(x2.dtype), x2.stride(0), int(cg or 0),
-              int(act_bits), int(swiglu), qw.data_ptr(), ldw, wbits, wscales.data_ptr(), *_bias_args(b),
-              y.data_ptr(), _lib.dtype_code(out_dtype), y.stride(0), m, n, k, work.data_ptr(), work.numel(),
-              _lib.stream_of(x2))
+    stream = _lib.stream_of_device(dev)
+    work = _linear_workspace(m, n, k, dev, stream)
+    bptr, bdt = (None, _lib.DT_BF16) if b is None else (b.data_ptr(), _lib.DTYPE_CODE[b.dtype])
+    _lib.call("mq_linear_rowscale", x2.data_ptr(), _lib.DTYPE_CODE[x2.dtype], 2 * k if swiglu else k, cg or 0, act_bits,
+              swiglu, qw.data_ptr(), ldw, wbits, wscales.data_ptr(), bptr, bdt, y.data_ptr(),
+              _lib.DTYPE_CODE[out_dtype], n, m, n, k, work.data_ptr(), work.numel(), stream)
     return y
 
 
@@ -657,7 +674,7 @@ def int8_rowscale_linear(x, q8, row_scale, bias=None, out_dtype=None, convrot_gr
         raise ValueError(f"Input K={k} does not match weight K={kw}")
     if convrot_groupsize and k % convrot_groupsize:
         raise ValueError(f"Input K={k} is not divisible by convrot_groupsize={convrot_groupsize}")
-    ws = row_scale.reshape(-1).to(torch.float32).contiguous()
+    ws = _row_scales(row_scale)
     if ws.numel() != n:
         raise ValueError(f"row scale must have {n} elements, got {ws.numel()}")
     y = _linear_rowscale(x, swiglu, convrot_groupsize, 8, q8, 8, ws, bias, n, k, _out_dtype(out_dtype, x_out))
