@@ -130,11 +130,11 @@ __device__ __forceinline__ void rotate_chunk_lds(float (&v)[16], const LdsTransp
     }
 }
 
-// am / L rounded to nearest for every am in [0, +inf] (L = 127 or 7) without a division: with
+// am / L rounded to nearest for every am in [0, +inf] (L = 127, 15 or 7) without a division: with
 // c = RN(1/L), q0 = RN(am c) is within an ulp of am / L, the residual am - q0 L is exact (one
 // fma), and RN(q0 + residual c) is the correctly rounded quotient (Markstein's correction step).
 // Checked bit for bit against the IEEE quotient for every non-negative float on the CPU
-// (tests/test_rotquant_scale.py). +inf, whose residual is NaN, is passed through.
+// (tests/test_rotquant_scale.py; as the fp16 scales of 15 and 7, tests/test_wquant_scale.py). +inf, whose residual is NaN, is passed through.
 template <int L>
 __device__ __forceinline__ float div_limit(float am) {
     constexpr float c = 1.0f / static_cast<float>(L);

@@ -15,12 +15,14 @@
 // where w is the rotated weight (the group formats are the configs' schemes, with the min / max code
 // choice of custom_nodes/comfy-lowbit-loader/formats.py:131-149 and the symmetric form of
 // tools/svdquant_probe.py:105-115; the row formats are tools/gptq_w4a4.py:197-203 and
-// tools/_formats.py:128-167). Scales and zero-points come from IEEE divisions. Codes take the
-// activation quantizer's product with the reciprocal and its exact division wherever that product
-// lies near a half-integer (quant16's argument: |w / s| < 128, here at most 127 or, for an fp16 scale
-// rounded down in its subnormal range, 23), so they are the IEEE quotient's codes.
+// tools/_formats.py:128-167). Scales are IEEE quotients (div_limit, checked for every
+// float). Codes and zero-points take the activation quantizer's product with the reciprocal and its
+// exact division wherever that product lies near a half-integer (quant16's argument: |w / s| < 128,
+// here at most 127 or, for an fp16 scale rounded down in its subnormal range, 23), so they are the
+// IEEE quotient's.
 //
-// What bounds it: HBM, 2.5 bytes per bf16 weight. At N = 12288, K = 3072 (96 MB): 26.5 us; one
+// What bounds it: HBM, 2.5 bytes per bf16 weight. At N = 12288, K = 3072 (96 MB): 22.4 us (26.5 with a
+// conversion, a compare and a shift per code and IEEE divisions per lane, when the VALU set it); one
 // workgroup per row with the row in LDS, a barrier per butterfly stage, one thread per group and
 // an IEEE division per weight took 142 us.
 #include "mq_device.h"
@@ -34,8 +36,6 @@ namespace mq {
 namespace {
 
 constexpr int kWaves = 4;   // wavefronts per workgroup
-
-__device__ __forceinline__ float clampf(float v, float lo, float hi) { return __builtin_fminf(__builtin_fmaxf(v, lo), hi); }
 
 // 16 consecutive weights of type DT at element i of w, as fp32; vec: 16-byte loads (the host has
 // checked the base and the row stride), else element by element.
@@ -89,34 +89,47 @@ __device__ __forceinline__ void rotate(float (&v)[16], const LdsTranspose& tr, i
     }
 }
 
-// rne(v / s) of 16 weights as floats, for |v / s| < 128 and r = recip_row(s): the rounded product,
-// or the IEEE quotient's rounding where the product lies near a half-integer (quant16).
-__device__ __forceinline__ void round16(const float (&v)[16], float r, float s, float (&n)[16]) {
+// kMagic + rne(v / s) of N values, for |v / s| < 128 and r = recip_row(s) (0 where every code is to be
+// 0): the rounded product, or the IEEE quotient's rounding where the product lies near a half-integer
+// (quant16). The integer sits in the low mantissa bits (two's complement), where the codes are clamped,
+// shifted by the zero-point (both exact) and packed from, with no conversion.
+template <int N>
+__device__ __forceinline__ void round_magic(const float (&v)[N], float r, float s, float (&m)[N]) {
     float dmax = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        n[j] = __builtin_fmaf(v[j], r, kMagic) - kMagic;
-        dmax = __builtin_fmaxf(dmax, __builtin_fabsf(__builtin_fmaf(v[j], r, -n[j])));
+    for (int j = 0; j < N; ++j) {
+        m[j] = __builtin_fmaf(v[j], r, kMagic);
+        dmax = __builtin_fmaxf(dmax, __builtin_fabsf(__builtin_fmaf(v[j], r, -(m[j] - kMagic))));
     }
     if (dmax > kTieWindow) {
 #pragma unroll
-        for (int j = 0; j < 16; ++j)
-            if (__builtin_fabsf(__builtin_fmaf(v[j], r, -n[j])) > kTieWindow) n[j] = __builtin_rintf(v[j] / s);
+        for (int j = 0; j < N; ++j)
+            if (__builtin_fabsf(__builtin_fmaf(v[j], r, -(m[j] - kMagic))) > kTieWindow)
+                m[j] = kMagic + __builtin_rintf(v[j] / s);
     }
 }
-
-// 16 codes (small integers as floats) as nibbles of two dwords, or as bytes of four.
-__device__ __forceinline__ uint32_t nibbles8(const float* c) {
-    uint32_t w = 0;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) w |= (static_cast<uint32_t>(static_cast<int>(c[e])) & 0xfu) << (4 * e);
-    return w;
+// kMagic + clamp(n, lo, hi) of kMagic + n; NaN gives lo, as fmin(fmax(NaN, lo), hi) does.
+__device__ __forceinline__ float clamp_magic(float m, float lo, float hi) {
+    return __builtin_amdgcn_fmed3f(m, kMagic + lo, kMagic + hi);
 }
-__device__ __forceinline__ uint32_t bytes4(const float* c) {
-    uint32_t w = 0;
+
+// The low bytes of four dwords as one, in order.
+__device__ __forceinline__ uint32_t low_bytes(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+    return __builtin_amdgcn_perm(b, a, 0x0c0c0400u) | __builtin_amdgcn_perm(d, c, 0x04000c0cu);
+}
+// 8 codes (magic-biased) as the nibbles of a dword, 4 codes as its bytes.
+template <bool SIGNED>
+__device__ __forceinline__ uint32_t nibbles8(const float* m) {
+    uint32_t t[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) w |= (static_cast<uint32_t>(static_cast<int>(c[e])) & 0xffu) << (8 * e);
-    return w;
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t even = __float_as_uint(m[2 * e]), odd = __float_as_uint(m[2 * e + 1]);
+        t[e] = (odd << 4) | (SIGNED ? even & 0xfu : even);   // (an unsigned code's low byte is the code)
+    }
+    return low_bytes(t[0], t[1], t[2], t[3]);
+}
+__device__ __forceinline__ uint32_t bytes4(const float* m) {
+    return low_bytes(__float_as_uint(m[0]), __float_as_uint(m[1]), __float_as_uint(m[2]), __float_as_uint(m[3]));
 }
 // 8 bytes of packed codes at p (4-byte aligned; wide: 8-byte aligned)
 __device__ __forceinline__ void store8(uint8_t* p, uint32_t lo, uint32_t hi, bool wide) {
@@ -151,7 +164,7 @@ wquant_group_kernel(const void* __restrict__ w, int64_t ldw, int64_t N, int K, i
         rotate(v, tr, hblock);
 
         // the group's extremes: 16 values here, then the four lanes that differ in lane bits 2 and 3
-        float s, z = 0.0f;
+        [[maybe_unused]] float lo = 0.0f;
         _Float16 h;
         if constexpr (FMT == 0) {
             float mn = v[0], mx = v[0];
@@ -164,27 +177,30 @@ wquant_group_kernel(const void* __restrict__ w, int64_t ldw, int64_t N, int K, i
             mx = __builtin_fmaxf(mx, dpp_mov<kRowRor4>(mx));
             mn = __builtin_fminf(mn, dpp_mov<kRowRor8>(mn));
             mx = __builtin_fmaxf(mx, dpp_mov<kRowRor8>(mx));
-            const float lo = __builtin_fminf(mn, 0.0f), hi = __builtin_fmaxf(mx, 0.0f);
-            h = static_cast<_Float16>((hi - lo) / 15.0f);
-            s = static_cast<float>(h);
-            z = s == 0.0f ? 0.0f : clampf(__builtin_rintf(-lo / s), 0.0f, 15.0f);
+            lo = __builtin_fminf(mn, 0.0f);
+            h = static_cast<_Float16>(div_limit<15>(__builtin_fmaxf(mx, 0.0f) - lo));
         } else {
             float am = 0.0f;
 #pragma unroll
             for (int e = 0; e < 16; ++e) am = __builtin_fmaxf(am, __builtin_fabsf(v[e]));
             am = __builtin_fmaxf(am, dpp_mov<kRowRor4>(am));
             am = __builtin_fmaxf(am, dpp_mov<kRowRor8>(am));
-            h = static_cast<_Float16>(am / 7.0f);
-            s = static_cast<float>(h);
+            h = static_cast<_Float16>(div_limit<7>(am));
         }
-        float c[16];
-        round16(v, recip_row(s), s, c);
+        const float s = static_cast<float>(h);
+        const float r = s == 0.0f ? 0.0f : recip_row(s);   // (a scale of 0: finite weights, codes and zero-point 0)
+        float z = 0.0f, c[16];
+        if constexpr (FMT == 0) {
+            const float t[1] = {-lo};
+            float m[1];
+            round_magic(t, r, s, m);
+            z = clamp_magic(m[0], 0.0f, 15.0f) - kMagic;
+        }
+        round_magic(v, r, s, c);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            c[e] = FMT == 0 ? clampf(c[e] + z, 0.0f, 15.0f) : clampf(c[e], -7.0f, 7.0f);
-            if (s == 0.0f) c[e] = 0.0f;
-        }
-        if (in) store8(q + row * ldq + col / 2, nibbles8(c), nibbles8(c + 8), wide);
+        for (int e = 0; e < 16; ++e)
+            c[e] = FMT == 0 ? clamp_magic(c[e] + z, 0.0f, 15.0f) : clamp_magic(c[e], -7.0f, 7.0f);
+        if (in) store8(q + row * ldq + col / 2, nibbles8<FMT == 1>(c), nibbles8<FMT == 1>(c + 8), wide);
         const bool lead = in && (lane & 12) == 0;   // one lane per group, of column col
         if (lead) {
             scale[row * ld_scale + col / 64] = __builtin_bit_cast(uint16_t, h);
@@ -238,11 +254,11 @@ wquant_row_kernel(const void* __restrict__ w, int64_t ldw, int K, int hblock, bo
         const int col = (i * kWaves + wave) * 1024 + 16 * seg;
         if (col >= K) continue;
         float c[16];
-        round16(v[i], r, s, c);
+        round_magic(v[i], r, s, c);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) c[e] = clampf(c[e], -L, L);
+        for (int e = 0; e < 16; ++e) c[e] = clamp_magic(c[e], -L, L);
         if constexpr (FMT == 2) {
-            store8(q + row * ldq + col / 2, nibbles8(c), nibbles8(c + 8), wide);
+            store8(q + row * ldq + col / 2, nibbles8<true>(c), nibbles8<true>(c + 8), wide);
         } else if (wide) {
             *reinterpret_cast<uint4*>(q + row * ldq + col) = uint4{bytes4(c), bytes4(c + 4), bytes4(c + 8), bytes4(c + 12)};
         } else {

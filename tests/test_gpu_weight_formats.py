@@ -74,6 +74,24 @@ def test_ties_and_small_scales(gpu_device):
     assert np.array_equal(q.cpu().numpy(), q0) and np.array_equal(s.cpu().numpy(), s0)
 
 
+def test_nan_and_infinite_weights(gpu_device):
+    """NaN weights are left out of the extremes and get the clamp's lower bound; an infinite weight makes a
+    row scale infinite and every finite code 0."""
+    print("[wquant] NaN, inf", flush=True)
+    w = torch.linspace(-1.0, 1.0, 256, device=gpu_device).repeat(4, 1)
+    clean = weights.quantize_w4a4_group_weight(w, 64, 0)
+    w[0, 5], w[1, 70] = float("nan"), float("nan")
+    q, s = weights.quantize_w4a4_group_weight(w, 64, 0)
+    q = q.view(torch.uint8)
+    assert torch.equal(s, clean[1]) and (int(q[0, 2]) >> 4) == 9 and (int(q[1, 35]) & 15) == 9     # -7
+    q, s, _ = weights.quantize_w4a8_asym_weight(w, 64, 0)
+    assert torch.isfinite(s).all() and (int(q[0, 2]) >> 4) == 0 and (int(q[1, 35]) & 15) == 0
+    w[2, 9] = float("inf")
+    q, s = weights.quantize_int8_convrot_weight(w, None)
+    assert int(q[0, 5]) == -127 and torch.isfinite(s[0]) and torch.isinf(s[2])
+    assert int(q[2, 9]) == -127 and int(q[2].abs().sum()) == 127
+
+
 def test_overflow_is_reported_once_per_call(gpu_device):
     w = torch.full((4, 2048), 1.0, device=gpu_device)
     w[3, 2000:] = 3.0e6
