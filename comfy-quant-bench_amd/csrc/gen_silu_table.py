@@ -106,9 +106,10 @@ def main_f16(path: str) -> None:
 
 def main(path: str) -> None:
     vals = table()
+    vals = [v for pair in zip(vals[:ENTRIES], vals[ENTRIES:]) for v in pair]   # the signs interleaved
     lines = [
         "// Generated by gen_silu_table.py: fp32 bits of silu(g) = g / (1 + exp(-g)), correctly rounded,",
-        f"// for bf16 gates with 0x{LO:04x} <= (bits & 0x7fff) < 0x{HI:04x}; index (|bits| - 0x{LO:04x}) + {ENTRIES} * sign.",
+        f"// for bf16 gates with 0x{LO:04x} <= (bits & 0x7fff) < 0x{HI:04x}; index 2 * (|bits| - 0x{LO:04x}) + sign.",
         "#pragma once",
         "#include <cstdint>",
         "namespace mq {",

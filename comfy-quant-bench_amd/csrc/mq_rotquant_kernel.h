@@ -16,17 +16,11 @@
 // column c has bits c0..c9; lane L of the wave loads the 16 consecutive columns of segment
 // s = (L >> 2) + 16 (L & 3) (two 16-byte bf16 loads), so register bits r0..r3 hold c0..c3 and
 // lane bits L0..L5 hold c8 c9 c4 c5 c6 c7. The radix-4 stages over (c0 c1) and (c2 c3) run in
-// registers. Plain inputs then move c4..c7 into the registers with a 16 x 16 transpose through LDS
-// (rotate_chunk_lds), run the stages over (c4 c5) and (c6 c7) there and transpose back, so the
-// exchanges cost no VALU instructions and the codes leave in the load layout. The SwiGLU kernels
-// exchange through lanes instead: the stage over (c4 c5) (blocks 64, 256) first swaps lane bits L2, L3 with register
-// bits r2, r3 through DPP row shifts written into the lanes of the receiving DPP banks only (one
-// v_mov_b32_dpp per moved value); the stage over (c6 c7) (block 256) swaps L4, L5 with r2, r3
-// through v_permlane16_swap / v_permlane32_swap (one instruction per register pair). Every
-// butterfly then runs in registers in the reference's order. After quantization four codes of
-// consecutive columns (r0 r1) sit in each dword; a final exchange of dwords across lane bits L2,
-// L3 gives every lane 16 consecutive codes, written with one 16-byte (int8) or 8-byte (packed
-// int4) store.
+// registers. A 16 x 16 transpose through LDS (rotate_chunk_lds) then moves c4..c7 into the registers, the
+// stages over (c4 c5) and (c6 c7) run there and the same transpose brings the load layout back, so the
+// exchanges cost no VALU instructions, every butterfly runs in registers in the reference's order, and
+// a lane's four dwords of codes are 16 consecutive columns, written with one 16-byte (int8) or 8-byte
+// (packed int4) store.
 //
 // Quantization without a per-element division: with r within 2^-23 relative of 1/s,
 // m = fma(v, r, 1.5*2^23) rounds v*r to an integer n. |v*r - v/s| < 2^-16 and
@@ -91,22 +85,23 @@ __device__ __forceinline__ void store_codes(bool nt, uint8_t* p, uint32_t w0, ui
 template <int IN>
 struct SiluF16Table;
 
+// The table's signs are interleaved: entry 2 j + sign for |bits| = kSiluLo + j.
 __device__ __forceinline__ float silu_f32(uint32_t b, float g, const float* tab) {
     const uint32_t t = b & 0x7fffu;
     const uint32_t j = __builtin_elementwise_min(t - kSiluLo, kSiluEntries - 1u);   // in bounds always
-    const uint32_t s = __float_as_uint(tab[j + ((b >> 15) << 12)]);
+    const uint32_t s = __float_as_uint(tab[2 * j + (b >> 15)]);
     const uint32_t big = (b >> 15) ? 0x80000000u : __float_as_uint(g);
     const uint32_t r = t < kSiluLo ? __float_as_uint(g * 0.5f) : s;
     return __uint_as_float(t >= kSiluLo + kSiluEntries ? big : r);
 }
 
-// Two activations from one dword of gates and one of ups (two bf16 each), as bf16-valued floats.
-// EAGER = false: bf16(silu(g) * u), one rounding (the fused quantizer). EAGER = true: silu(g) is
-// rounded to bf16 first and the product (exact in fp32: two 8-bit significands) then rounded again,
-// bf16(bf16(silu(g)) * u): the eager torch path silu(gate).mul_(up) in bf16.
+// The activation of one pair from silu of its gates (s0, s1) and the dword of its ups (two bf16 each), as
+// bf16-valued floats. EAGER = false: bf16(silu(g) * u), one rounding (the fused quantizer).
+// EAGER = true: silu(g) is rounded to bf16 first and the product (exact in fp32: two 8-bit
+// significands) then rounded again, bf16(bf16(silu(g)) * u): the eager torch path silu(gate).mul_(up)
+// in bf16.
 template <bool EAGER>
-__device__ __forceinline__ void swiglu_pair(uint32_t wg, uint32_t wu, const float* tab, float& a0, float& a1) {
-    float s0 = silu_f32(wg & 0xffffu, bf16lo(wg), tab), s1 = silu_f32(wg >> 16, bf16hi(wg), tab);
+__device__ __forceinline__ void swiglu_product(float s0, float s1, uint32_t wu, float& a0, float& a1) {
     if constexpr (EAGER) {
         const uint32_t sh = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{s0, s1}, bf16x2));
         s0 = __uint_as_float(sh << 16);
@@ -117,6 +112,42 @@ __device__ __forceinline__ void swiglu_pair(uint32_t wg, uint32_t wu, const floa
     const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{p0, p1}, bf16x2));
     a0 = __uint_as_float(h << 16);
     a1 = __uint_as_float(h & 0xffff0000u);
+}
+
+// 16 activations from their gates and ups. Nearly every gate lies in the table's range, so all are
+// looked up, two at a time in 16-bit halves: y = bits - kSiluLo holds the sign in bit 15 and, in range, j
+// in bits 0 - 11 and zeros in bits 12 - 14 (outside it, some of those are set: kSiluLo is 0x3300 and the
+// table ends at 0x4300), and 8 j + 4 sign, masked into the table whatever y is, is the entry's byte.
+// `out` gathers the y; a lane that finds kSiluOut bits in it forms its values again with silu_f32's closed
+// forms (once for all its chunks, so that their lookups overlap). 7 VALU instructions an element
+// instead of 16, in kernels that the VALU sets; with the rotation's exchanges through LDS instead of
+// lane swaps (4 more): M = 4096, K = 12288, packed int4 59.4 -> 51.1 us (226 MB); M = 32760, K = 3072, int8
+// 126 -> 106 us. (Few long rows gain nothing: M = 16, K = 12288 7.9 -> 8.1 us, latency.)
+constexpr uint32_t kSiluOut = 0x70007000u;
+template <bool EAGER>
+__device__ __forceinline__ void swiglu_lookup(const uint32_t (&w)[8], const uint32_t (&wu)[8], const float* tab,
+                                              float (&v)[16], uint32_t& out) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    static_assert(kSiluLo == 0x3300u && kSiluEntries == 4096u, "the range test's bits");
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const u16x2 y = __builtin_bit_cast(u16x2, w[j]) - static_cast<uint16_t>(kSiluLo);
+        out |= __builtin_bit_cast(uint32_t, y);
+        const uint32_t at = (__builtin_bit_cast(uint32_t, static_cast<u16x2>(y << 3)) & 0x7ff87ff8u) |
+                            (__builtin_bit_cast(uint32_t, static_cast<u16x2>(y >> 13)) & 0x00040004u);
+        const char* t = reinterpret_cast<const char*>(tab);
+        const float s0 = *reinterpret_cast<const float*>(t + (at & 0xffffu));
+        const float s1 = *reinterpret_cast<const float*>(t + (at >> 16));
+        swiglu_product<EAGER>(s0, s1, wu[j], v[2 * j], v[2 * j + 1]);
+    }
+}
+template <bool EAGER>
+__device__ __forceinline__ void swiglu_any(const uint32_t (&w)[8], const uint32_t (&wu)[8], const float* tab,
+                                           float (&v)[16]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        swiglu_product<EAGER>(silu_f32(w[j] & 0xffffu, bf16lo(w[j]), tab), silu_f32(w[j] >> 16, bf16hi(w[j]), tab), wu[j],
+                              v[2 * j], v[2 * j + 1]);
 }
 
 // fp16 inputs: silu of both gates from the global fp16 table, the products rounded to fp16 (EAGER:
@@ -136,6 +167,13 @@ __device__ __forceinline__ void swiglu_pair_f16(uint32_t wg, uint32_t wu, const 
     a1 = f16hi(h);
 }
 
+// 16 consecutive 16-bit values (16-byte aligned), two per dword.
+__device__ __forceinline__ void load16bits(const uint16_t* p, uint32_t (&w)[8]) {
+    const uint4 a = *reinterpret_cast<const uint4*>(p), b = *reinterpret_cast<const uint4*>(p + 8);
+    w[0] = a.x; w[1] = a.y; w[2] = a.z; w[3] = a.w;
+    w[4] = b.x; w[5] = b.y; w[6] = b.z; w[7] = b.w;
+}
+
 // OUT: 0 = int8 codes, 1 = int4 codes one per byte, 2 = int4 codes packed two per byte,
 //      3 = int4 codes one per byte as 16 * q, negated in odd 64-column groups (the operand layout
 //          the group-scale GEMM takes for int4 activations: exact, and 16x finer in its fp32 step).
@@ -152,16 +190,11 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
                 uint8_t* __restrict__ q, int64_t ldq, float* __restrict__ scale, bool nt) {
     constexpr int LIMIT = OUT == 0 ? 127 : 7;
     constexpr int RPG = kWaves / W;                      // rows per workgroup step
-    // Plain inputs exchange lanes and registers through LDS (rotate_chunk_lds) and leave the
-    // rotation in the load layout; the SwiGLU prologue, whose LDS holds its silu table, keeps the
-    // lane swaps. LB: the block whose register layout the rotated values are in.
-    constexpr bool kLdsT = ACT == 0 && BLK >= 64;
-    constexpr int LB = kLdsT ? 16 : BLK;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int wr = wave % W;                             // this wave's share of its row
     [[maybe_unused]] LdsTranspose tr{nullptr, nullptr};
-    if constexpr (kLdsT) {
+    if constexpr (BLK >= 64) {
         __shared__ __attribute__((aligned(16))) float tr_lds[kWaves * kTrWave];
         float* base = tr_lds + wave * kTrWave + (lane & 3) * kTrG;
         tr.w = base + (lane >> 2);
@@ -182,9 +215,7 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
         __shared__ float red_lds[2][kWaves];
         red = &red_lds[0][0];
     }
-    const int seg_ld = (lane >> 2) + 16 * (lane & 3);   // 16-column segment this lane loads
-    // after the final dword exchange a lane holds the 16 codes of segment seg_st
-    const int seg_st = LB >= 256 ? (lane >> 4) + 4 * ((lane >> 2) & 3) + 16 * (lane & 3) : seg_ld;
+    const int seg = (lane >> 2) + 16 * (lane & 3);   // 16-column segment this lane loads, rotates and stores
     const int64_t groups = (static_cast<int64_t>(M) + RPG - 1) / RPG;
     int parity = 0;
     // every wave runs the same number of steps (the bound is uniform over the workgroup), so the
@@ -206,9 +237,10 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
 
         float v[NCH][16];
         bool in[NCH];
+        [[maybe_unused]] uint32_t silu_out = 0u;
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
-            const int e0 = (c * W + wr) * 1024 + seg_ld * 16;
+            const int e0 = (c * W + wr) * 1024 + seg * 16;
             in[c] = e0 < K;
             const int e = in[c] ? e0 : 0;
             if constexpr (IN == 2) {
@@ -223,17 +255,17 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
                 }
                 continue;
             }
-            const uint4 a = *reinterpret_cast<const uint4*>(xr + e);
-            const uint4 b = *reinterpret_cast<const uint4*>(xr + e + 8);
-            const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            uint32_t w[8];
+            load16bits(xr + e, w);
             if constexpr (ACT >= 1) {
-                const uint4 ua = *reinterpret_cast<const uint4*>(xr + K + e);
-                const uint4 ub = *reinterpret_cast<const uint4*>(xr + K + e + 8);
-                const uint32_t wu[8] = {ua.x, ua.y, ua.z, ua.w, ub.x, ub.y, ub.z, ub.w};
+                uint32_t wu[8];
+                load16bits(xr + K + e, wu);
+                if constexpr (IN == 1) {
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    if constexpr (IN == 1) swiglu_pair_f16<ACT == 2>(w[j], wu[j], tab16, v[c][2 * j], v[c][2 * j + 1]);
-                    else swiglu_pair<ACT == 2>(w[j], wu[j], tab, v[c][2 * j], v[c][2 * j + 1]);
+                    for (int j = 0; j < 8; ++j)
+                        swiglu_pair_f16<ACT == 2>(w[j], wu[j], tab16, v[c][2 * j], v[c][2 * j + 1]);
+                } else {
+                    swiglu_lookup<ACT == 2>(w, wu, tab, v[c], silu_out);
                 }
             } else {
 #pragma unroll
@@ -244,11 +276,23 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
             }
         }
 
+        if constexpr (ACT >= 1 && IN == 0) {
+            if (silu_out & kSiluOut) {   // a gate outside the table: the lane's values again, in full
+#pragma unroll
+                for (int c = 0; c < NCH; ++c) {
+                    const int e = in[c] ? (c * W + wr) * 1024 + seg * 16 : 0;
+                    uint32_t w[8], wu[8];
+                    load16bits(xr + e, w);
+                    load16bits(xr + K + e, wu);
+                    swiglu_any<ACT == 2>(w, wu, tab, v[c]);
+                }
+            }
+        }
+
         float am = 0.0f;
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
-            if constexpr (kLdsT) rotate_chunk_lds<BLK>(v[c], tr);
-            else rotate_chunk<BLK>(v[c], lane);
+            rotate_chunk_lds<BLK>(v[c], tr);
             float amc = 0.0f;
 #pragma unroll
             for (int j = 0; j < 16; ++j) amc = __builtin_fmaxf(amc, __builtin_fabsf(v[c][j]));
@@ -275,20 +319,14 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
             // quantization is odd-symmetric (rint and the clamp are), so negating the input of an
-            // odd 64-column group negates its codes exactly; in the block-256 lane-swap layout the
-            // group parity is register bit r2, so the sign applies per dword below instead
+            // odd 64-column group (column bit 6 is lane bit 4) negates its codes exactly
             float mq[16];
-            quant16<LIMIT>(v[c], OUT == 3 && LB < 256 && col_bit6<LB>(lane, 0) ? -1.0f : 1.0f, r, s, mq);
+            quant16<LIMIT>(v[c], OUT == 3 && ((lane >> 4) & 1) ? -1.0f : 1.0f, r, s, mq);
             uint32_t word[4];
 #pragma unroll
             for (int hi = 0; hi < 4; ++hi) {
                 uint32_t m0 = __float_as_uint(mq[4 * hi + 0]), m1 = __float_as_uint(mq[4 * hi + 1]);
                 uint32_t m2 = __float_as_uint(mq[4 * hi + 2]), m3 = __float_as_uint(mq[4 * hi + 3]);
-                if constexpr (OUT == 3 && LB >= 256) {
-                    if (col_bit6<LB>(lane, 4 * hi)) {   // negate the four codes (two's complement bytes)
-                        m0 = -m0; m1 = -m1; m2 = -m2; m3 = -m3;
-                    }
-                }
                 if constexpr (OUT == 3) {
                     m0 <<= 4; m1 <<= 4; m2 <<= 4; m3 <<= 4;
                 }
@@ -300,13 +338,7 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
                     word[hi] = lo16 | hi16;
                 }
             }
-            // dword index bits hold (c6 c7) for block 256 and (c4 c5) for block 64; lane bits
-            // L2 L3 hold (c2 c3): exchange them so each lane's four dwords are consecutive columns
-            if constexpr (LB >= 64) {
-                swap_lane_reg<2, 0>(word, lane);
-                swap_lane_reg<3, 1>(word, lane);
-            }
-            const int col = (c * W + wr) * 1024 + seg_st * 16;
+            const int col = (c * W + wr) * 1024 + seg * 16;
             if (col >= K) continue;
             if constexpr (OUT == 2)
                 store_codes(nt, qr + col / 2, word[0] | (word[1] << 16), word[2] | (word[3] << 16));
