@@ -415,7 +415,7 @@ def expand_w4_weight(qweight: torch.Tensor, wzeros=None, layout: int = _lib.ACT_
 
 # The linears run their 4-bit weights from an int8 expansion wherever the packed weights would run
 # on the wide kernel too, so that the results are the same bits either way: group scales above 128
-# rows (fewer rows run on the 128 x 128 few-row kernel, whose group epilogue rounds differently),
+# rows (fewer rows run on the few-row kernel, whose group epilogue rounds differently),
 # row scales above the GEMV's 4 rows (exact int32 sums on every kernel). The GEMV reads the packed
 # bytes: it is bound by their HBM traffic. The expansion is made on a weight's first such call and
 # kept until the tensor it was made from (its base tensor, for a view) is freed, for as long as that
