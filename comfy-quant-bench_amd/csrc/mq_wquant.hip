@@ -327,52 +327,82 @@ __global__ void __launch_bounds__(256) tile16_kernel(const uint8_t* w, int64_t l
     }
 }
 
-// Packed 4-bit weights [N, K/2] (row stride ldw bytes) expanded to int8 in the same 16-row tiles,
-// one thread per 16-byte unit as in tile16_kernel. A unit holds 16 consecutive k of one row and
-// K group g (its 8 packed bytes); value v = q - z (uint4 with zero-point nibble z of group g) or
-// the signed nibble, then by layout: 0 (the group GEMM's int8 activation layout) negated in odd
-// groups, 2 (its x16 int4 layout) 16 * v for signed weights, 3 (row scale) v as it is.
-__global__ void __launch_bounds__(256) expand_w4_kernel(const uint8_t* qw, int64_t ldw, const uint8_t* wz,
-                                                       int64_t ldwz, int64_t N, int64_t K, int layout,
-                                                       uint8_t* out) {
-    const int64_t G = K / 64, units = (N + 15) / 16 * 16 * (K / 16);
-    for (int64_t u = blockIdx.x * int64_t(256) + threadIdx.x; u < units; u += int64_t(gridDim.x) * 256) {
-        const int64_t chunk = u & 3, row = (u >> 2) & 15, g = (u >> 6) % G, band = (u >> 6) / G;
-        const int64_t n = band * 16 + row;
+// Packed 4-bit weights [N, K/2] (row stride ldw bytes) expanded to int8 in the same 16-row tiles. One
+// wavefront per tile (band, K group g), a lane per row and 16-column chunk (8 packed bytes in, 16 out);
+// value v = q - z (uint4 with zero-point nibble z of group g) or the signed nibble, then by layout: 0
+// (the group GEMM's int8 activation layout) negated in odd groups, 2 (its x16 int4 layout) 16 * v for
+// signed weights, 3 (row scale) v as it is. Four values at a time, as the wide GEMM unpacks packed
+// weights: (q + 0x80 - z) ^ 0x80 per byte, or (0x80 + z - q) ^ 0x80 negated, without inter-byte carries,
+// and two byte permutes back to k order. Eight masked adds per 16 values instead of
+// about six operations a value, no 64-bit division per thread: HBM-bound, where the byte at a time it replaces
+// was bound by its VALU work. With the scales' launch below, [12288, 3072] uint4 takes 18-19.5 us (26.4 before;
+// its 60 MB take 12 at the rate of a large copy), [3072, 14336] 18.4 (28.7), row-scale [3072, 12288] 11.4 (19.4).
+enum ExpandKind : int { kExpandU4 = 0, kExpandI4 = 1, kExpandI4x16 = 2 };
+template <int KIND>
+__global__ void __launch_bounds__(64 * kWaves)
+expand_w4_kernel(const uint8_t* __restrict__ qw, int64_t ldw, const uint8_t* __restrict__ wz, int64_t ldwz, int64_t N,
+                 int G, bool alternate, uint8_t* __restrict__ out) {
+    const int lane = threadIdx.x & 63, chunk = lane & 3;
+    const int64_t tiles = (N + 15) / 16 * G;
+    for (int64_t t = static_cast<int64_t>(blockIdx.x) * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); t < tiles;
+         t += static_cast<int64_t>(gridDim.x) * kWaves) {
+        const int64_t band = t / G;
+        const int g = static_cast<int>(t - band * G);
+        const int64_t n = band * 16 + (lane >> 2);
         uint32_t o[4] = {0u, 0u, 0u, 0u};
         if (n < N) {
-            const uint2 w = *reinterpret_cast<const uint2*>(qw + n * ldw + g * 32 + chunk * 8);
-            const int z = wz ? (wz[n * ldwz + (g >> 1)] >> (4 * (g & 1))) & 15 : 0;
-            const bool neg = layout == 0 && (g & 1);
+            const uint2 w2 = *reinterpret_cast<const uint2*>(qw + n * ldw + g * 32 + chunk * 8);
+            uint32_t z = 8u;
+            if constexpr (KIND == kExpandU4) z = (wz[n * ldwz + (g >> 1)] >> (4 * (g & 1))) & 15u;
+            const bool neg = alternate && (g & 1);
+            const uint32_t zz = z * 0x01010101u;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const uint32_t byte = (e < 8 ? w.x >> (8 * (e >> 1)) : w.y >> (8 * ((e - 8) >> 1))) & 0xffu;
-                const int q = (byte >> (4 * (e & 1))) & 15;
-                int v = wz ? q - z : (q >= 8 ? q - 16 : q);
-                if (neg) v = -v;
-                if (layout == 2 && !wz) v *= 16;
-                o[e >> 2] |= (static_cast<uint32_t>(v) & 0xffu) << (8 * (e & 3));
+            for (int h = 0; h < 2; ++h) {
+                uint32_t w = h ? w2.y : w2.x, lo, hi;
+                if constexpr (KIND == kExpandI4x16) {
+                    lo = (w << 4) & 0xf0f0f0f0u;
+                    hi = w & 0xf0f0f0f0u;
+                } else {
+                    if constexpr (KIND == kExpandI4) w ^= 0x88888888u;   // v + 8
+                    lo = w & 0x0f0f0f0fu;
+                    hi = (w >> 4) & 0x0f0f0f0fu;
+                    if (neg) {
+                        lo = ((0x80808080u | zz) - lo) ^ 0x80808080u;
+                        hi = ((0x80808080u | zz) - hi) ^ 0x80808080u;
+                    } else {
+                        lo = (lo + (0x80808080u - zz)) ^ 0x80808080u;
+                        hi = (hi + (0x80808080u - zz)) ^ 0x80808080u;
+                    }
+                }
+                o[2 * h] = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
+                o[2 * h + 1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
             }
         }
-        *reinterpret_cast<uint4*>(out + u * 16) = make_uint4(o[0], o[1], o[2], o[3]);
+        *reinterpret_cast<uint4*>(out + t * 1024 + lane * 16) = make_uint4(o[0], o[1], o[2], o[3]);
     }
 }
 
 // fp16 group scales [N, G] (row stride ldws) as the expanded-weight group GEMM's lanes load them:
 // dword [g][c][u] (u fastest, ld dwords per [g][c]) = ws[32 u + c, g] | ws[32 u + 16 + c, g] << 16,
-// zero for columns past N and groups past G; G4 groups in all (G rounded up to four).
-__global__ void __launch_bounds__(256) expand_scales_kernel(const uint16_t* ws, int64_t ldws, int64_t N, int64_t G,
-                                                           int64_t G4, int64_t ld, uint32_t* out) {
-    const int64_t total = G4 * 16 * ld;
-    for (int64_t i = blockIdx.x * int64_t(256) + threadIdx.x; i < total; i += int64_t(gridDim.x) * 256) {
-        const int64_t u = i % ld, c = (i / ld) % 16, g = i / (16 * ld);
-        const int64_t n0 = 32 * u + c, n1 = n0 + 16;
+// zero for columns past N and groups past G; G4 groups in all (G rounded up to four). A thread takes four
+// groups of one (c, u): eight consecutive bytes of each of its two rows (one cache line, where a thread per
+// group fetched the line again), and stores that run along u.
+__global__ void __launch_bounds__(256) expand_scales_kernel(const uint16_t* __restrict__ ws, int64_t ldws, int64_t N,
+                                                           int G, int ld, uint32_t* __restrict__ out) {
+    const int ublocks = (ld + 255) / 256;
+    const int cg = blockIdx.x / ublocks, c = cg & 15, g0 = cg / 16 * 4;
+    const int u = (blockIdx.x - cg * ublocks) * 256 + threadIdx.x;
+    if (u >= ld) return;
+    const int64_t n0 = 32 * static_cast<int64_t>(u) + c, n1 = n0 + 16;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int g = g0 + i;
         uint32_t v = 0u;
         if (g < G) {
             if (n0 < N) v = ws[n0 * ldws + g];
             if (n1 < N) v |= static_cast<uint32_t>(ws[n1 * ldws + g]) << 16;
         }
-        out[i] = v;
+        out[(static_cast<int64_t>(g) * 16 + c) * ld + u] = v;
     }
 }
 
@@ -380,19 +410,26 @@ __global__ void __launch_bounds__(256) expand_scales_kernel(const uint16_t* ws, 
 
 int launch_expand_scales_w4(const uint16_t* ws, int64_t ldws, int64_t N, int64_t K, uint32_t* out,
                             hipStream_t stream) {
-    const int64_t G = K / 64, G4 = (G + 3) / 4 * 4, ld = scale_pair_ld(N);
-    const int64_t blocks = std::min<int64_t>((G4 * 16 * ld + 255) / 256, 65536);
-    hipLaunchKernelGGL(expand_scales_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, ws, ldws, N, G,
-                       G4, ld, out);
+    // One block index over (four groups, c, 256 u): G runs past a grid's 65535 in y and z for one long row. The
+    // expansion is under 2 GiB, which keeps the threads under 2^31.
+    const int64_t G = K / 64, ld = scale_pair_ld(N), blocks = (G + 3) / 4 * 16 * ((ld + 255) / 256);
+    hipLaunchKernelGGL(expand_scales_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, ws, ldws, N,
+                       static_cast<int>(G), static_cast<int>(ld), out);
     return launch_status("expand_scales_w4");
 }
 
 int launch_expand_weight_w4(const uint8_t* qw, int64_t ldw, const uint8_t* wz, int64_t ldwz, int64_t N, int64_t K,
                             int layout, uint8_t* out, hipStream_t stream) {
-    const int64_t units = (N + 15) / 16 * 16 * (K / 16);
-    const int64_t blocks = std::min<int64_t>((units + 255) / 256, 65536);
-    hipLaunchKernelGGL(expand_w4_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, qw, ldw, wz, ldwz,
-                       N, K, layout, out);
+    const int G = static_cast<int>(K / 64);
+    const int64_t tiles = (N + 15) / 16 * G;
+    const dim3 grid(static_cast<unsigned>(std::min<int64_t>((tiles + kWaves - 1) / kWaves, int64_t(1) << 20)));
+    const bool alternate = layout == 0;
+#define MQ_EX(KIND) \
+    hipLaunchKernelGGL(expand_w4_kernel<KIND>, grid, dim3(64 * kWaves), 0, stream, qw, ldw, wz, ldwz, N, G, alternate, out)
+    if (wz) MQ_EX(kExpandU4);
+    else if (layout == 2) MQ_EX(kExpandI4x16);
+    else MQ_EX(kExpandI4);
+#undef MQ_EX
     return launch_status("expand_weight_w4");
 }
 
