@@ -333,9 +333,9 @@ __global__ void __launch_bounds__(256) tile16_kernel(const uint8_t* w, int64_t l
 // (the group GEMM's int8 activation layout) negated in odd groups, 2 (its x16 int4 layout) 16 * v for
 // signed weights, 3 (row scale) v as it is. Four values at a time, as the wide GEMM unpacks packed
 // weights: (q + 0x80 - z) ^ 0x80 per byte, or (0x80 + z - q) ^ 0x80 negated, without inter-byte carries,
-// and two byte permutes back to k order. Eight masked adds per 16 values instead of
-// about six operations a value, no 64-bit division per thread: HBM-bound, where the byte at a time it replaces
-// was bound by its VALU work. With the scales' launch below, [12288, 3072] uint4 takes 18-19.5 us (26.4 before;
+// and two byte permutes back to k order: about two operations a value where the value at a time it
+// replaces, bound by its VALU work, took six and two 64-bit divisions a thread (the expansion is under 2 GiB, so
+// the tiles count in 32 bits and the division is one per wave). With the scales' launch below, [12288, 3072] uint4 takes 18-19.5 us (26.4 before;
 // its 60 MB take 12 at the rate of a large copy), [3072, 14336] 18.4 (28.7), row-scale [3072, 12288] 11.4 (19.4).
 enum ExpandKind : int { kExpandU4 = 0, kExpandI4 = 1, kExpandI4x16 = 2 };
 template <int KIND>
@@ -343,12 +343,11 @@ __global__ void __launch_bounds__(64 * kWaves)
 expand_w4_kernel(const uint8_t* __restrict__ qw, int64_t ldw, const uint8_t* __restrict__ wz, int64_t ldwz, int64_t N,
                  int G, bool alternate, uint8_t* __restrict__ out) {
     const int lane = threadIdx.x & 63, chunk = lane & 3;
-    const int64_t tiles = (N + 15) / 16 * G;
-    for (int64_t t = static_cast<int64_t>(blockIdx.x) * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); t < tiles;
-         t += static_cast<int64_t>(gridDim.x) * kWaves) {
-        const int64_t band = t / G;
-        const int g = static_cast<int>(t - band * G);
-        const int64_t n = band * 16 + (lane >> 2);
+    const int tiles = static_cast<int>((N + 15) / 16) * G;
+    const int t = blockIdx.x * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (t < tiles) {
+        const int band = t / G, g = t - band * G;
+        const int64_t n = static_cast<int64_t>(band) * 16 + (lane >> 2);
         uint32_t o[4] = {0u, 0u, 0u, 0u};
         if (n < N) {
             const uint2 w2 = *reinterpret_cast<const uint2*>(qw + n * ldw + g * 32 + chunk * 8);
@@ -378,7 +377,7 @@ expand_w4_kernel(const uint8_t* __restrict__ qw, int64_t ldw, const uint8_t* __r
                 o[2 * h + 1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
             }
         }
-        *reinterpret_cast<uint4*>(out + t * 1024 + lane * 16) = make_uint4(o[0], o[1], o[2], o[3]);
+        *reinterpret_cast<uint4*>(out + static_cast<int64_t>(t) * 1024 + lane * 16) = make_uint4(o[0], o[1], o[2], o[3]);
     }
 }
 
@@ -422,7 +421,7 @@ int launch_expand_weight_w4(const uint8_t* qw, int64_t ldw, const uint8_t* wz, i
                             int layout, uint8_t* out, hipStream_t stream) {
     const int G = static_cast<int>(K / 64);
     const int64_t tiles = (N + 15) / 16 * G;
-    const dim3 grid(static_cast<unsigned>(std::min<int64_t>((tiles + kWaves - 1) / kWaves, int64_t(1) << 20)));
+    const dim3 grid(static_cast<unsigned>((tiles + kWaves - 1) / kWaves));   // tiles < 2 GiB / 1 KiB
     const bool alternate = layout == 0;
 #define MQ_EX(KIND) \
     hipLaunchKernelGGL(expand_w4_kernel<KIND>, grid, dim3(64 * kWaves), 0, stream, qw, ldw, wz, ldwz, N, G, alternate, out)
