@@ -184,14 +184,20 @@ __device__ __forceinline__ void load16bits(const uint16_t* p, uint32_t (&w)[8]) 
 // NCH: chunks per wave; W: waves per row (NCH * W * 1024 >= K).
 // TL: codes in 16-row tiles (one code per byte only), chosen at compile time so that the
 // row-major store keeps its exact code
-template <int BLK, int OUT, int NCH, int ACT, int W, int IN, bool TL>
+// DEAD: rows whose chunks leave at least one wave without a last chunk (chosen by the host, W > 1): a
+// chunk wholly past K is loaded, in bounds, so that the loads stay together, and then neither rotated
+// nor quantized. Row-major codes, M = 32760: K = 14336 (two of 16 chunks) 282 -> 271 us, K = 5120 118 ->
+// 101; M = 4096, K = 9216 26.1 -> 23.1. Rows that fill their chunks keep the code without the test: with
+// it an int8 linear of K = 12288, M = 4096 took 150.3 us for 149.4 on the same device.
+template <int BLK, int OUT, int NCH, int ACT, int W, int IN, bool TL, bool DEAD>
 __global__ void __launch_bounds__(64 * kWaves)
 rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
                 uint8_t* __restrict__ q, int64_t ldq, float* __restrict__ scale, bool nt) {
     constexpr int LIMIT = OUT == 0 ? 127 : 7;
     constexpr int RPG = kWaves / W;                      // rows per workgroup step
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int wave = threadIdx.x >> 6;
+    if constexpr (DEAD) wave = __builtin_amdgcn_readfirstlane(wave);
     const int wr = wave % W;                             // this wave's share of its row
     [[maybe_unused]] LdsTranspose tr{nullptr, nullptr};
     if constexpr (BLK >= 64) {
@@ -216,10 +222,8 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
         red = &red_lds[0][0];
     }
     const int seg = (lane >> 2) + 16 * (lane & 3);   // 16-column segment this lane loads, rotates and stores
-    // whether this wave's last chunk lies in the row at all (the earlier ones always do): a chunk wholly
-    // past K is loaded, in bounds, so that the loads stay together, and then left (K = 14336: two of 16
-    // chunks; M = 32760 283 -> 273 us; K = 9216, M = 4096 26.3 -> 23.0 us)
-    const bool last = ((NCH - 1) * W + wr) * 1024 < K;
+    [[maybe_unused]] bool last = true;                   // whether this wave's last chunk lies in the row
+    if constexpr (DEAD) last = ((NCH - 1) * W + wr) * 1024 < K;
     const int64_t groups = (static_cast<int64_t>(M) + RPG - 1) / RPG;
     int parity = 0;
     // every wave runs the same number of steps (the bound is uniform over the workgroup), so the
@@ -296,7 +300,7 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
         float am = 0.0f;
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
-            if (c == NCH - 1 && !last) break;
+            if (DEAD && c == NCH - 1 && !last) break;
             rotate_chunk_lds<BLK>(v[c], tr);
             float amc = 0.0f;
 #pragma unroll
@@ -323,7 +327,7 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
         uint8_t* qr = tiled ? q + (row >> 4) * (static_cast<int64_t>(K) << 4) + (row & 15) * 64 : q + row * ldq;
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
-            if (c == NCH - 1 && !last) break;
+            if (DEAD && c == NCH - 1 && !last) break;
             // quantization is odd-symmetric (rint and the clamp are), so negating the input of an
             // odd 64-column group (column bit 6 is lane bit 4) negates its codes exactly
             float mq[16];
@@ -370,7 +374,7 @@ int launch_rq(const uint16_t* x, int64_t M, int64_t K, int64_t ldx, void* q, int
         int per_cu = per_cu_cache.load(std::memory_order_relaxed);
         if (per_cu <= 0) {
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &per_cu, reinterpret_cast<const void*>(&rotquant_kernel<BLK, OUT, NCH, ACT, W, IN, false>),
+                    &per_cu, reinterpret_cast<const void*>(&rotquant_kernel<BLK, OUT, NCH, ACT, W, IN, false, false>),
                     64 * kWaves,
                     0) != hipSuccess ||
                 per_cu <= 0)
@@ -383,15 +387,18 @@ int launch_rq(const uint16_t* x, int64_t M, int64_t K, int64_t ldx, void* q, int
     }
     if (wgs == 0) return 0;
     const bool nt = (OUT == 2 ? M * K / 2 : M * K) >= kNtCodeBytes;
+    const bool dead = W > 1 && K <= (NCH * W - 1) * 1024;
     // a row stride of 0 asks for the codes in 16-row tiles (one code per byte)
-    if (OUT != 2 && ldq == 0)
-        hipLaunchKernelGGL((rotquant_kernel<BLK, OUT, NCH, ACT, W, IN, OUT != 2>), dim3(static_cast<unsigned>(wgs)),
-                           dim3(64 * kWaves), 0, stream, x, ldx, static_cast<int>(M), static_cast<int>(K),
-                           static_cast<uint8_t*>(q), ldq, scale, nt);
-    else
-        hipLaunchKernelGGL((rotquant_kernel<BLK, OUT, NCH, ACT, W, IN, false>), dim3(static_cast<unsigned>(wgs)),
-                           dim3(64 * kWaves), 0, stream, x, ldx, static_cast<int>(M), static_cast<int>(K),
-                           static_cast<uint8_t*>(q), ldq, scale, nt);
+    const bool tiled = OUT != 2 && ldq == 0;
+#define MQ_RQ(TL, DEAD)                                                                                             \
+    hipLaunchKernelGGL((rotquant_kernel<BLK, OUT, NCH, ACT, W, IN, TL, DEAD>), dim3(static_cast<unsigned>(wgs)),     \
+                       dim3(64 * kWaves), 0, stream, x, ldx, static_cast<int>(M), static_cast<int>(K),              \
+                       static_cast<uint8_t*>(q), ldq, scale, nt)
+    if (tiled && dead) MQ_RQ(OUT != 2, (W > 1));
+    else if (tiled) MQ_RQ(OUT != 2, false);
+    else if (dead) MQ_RQ(false, (W > 1));
+    else MQ_RQ(false, false);
+#undef MQ_RQ
     return launch_status("rotquant");
 }
 
