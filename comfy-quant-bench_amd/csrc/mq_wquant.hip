@@ -188,7 +188,7 @@ wquant_group_kernel(const void* __restrict__ w, int64_t ldw, int64_t N, int K, i
             h = static_cast<_Float16>(div_limit<7>(am));
         }
         const float s = static_cast<float>(h);
-        const float r = s == 0.0f ? 0.0f : recip_row(s);   // (a scale of 0: finite weights, codes and zero-point 0)
+        const float r = s == 0.0f ? 0.0f : recip_row(s);   // (a scale of 0: codes and zero-point 0)
         float z = 0.0f, c[16];
         if constexpr (FMT == 0) {
             const float t[1] = {-lo};
@@ -197,9 +197,11 @@ wquant_group_kernel(const void* __restrict__ w, int64_t ldw, int64_t N, int K, i
             z = clamp_magic(m[0], 0.0f, 15.0f) - kMagic;
         }
         round_magic(v, r, s, c);
+        // (a NaN weight gets the lower bound: 0 where the scale is 0, as every other code of that group)
+        const float lim = s == 0.0f ? 0.0f : 7.0f;
 #pragma unroll
         for (int e = 0; e < 16; ++e)
-            c[e] = FMT == 0 ? clamp_magic(c[e] + z, 0.0f, 15.0f) : clamp_magic(c[e], -7.0f, 7.0f);
+            c[e] = FMT == 0 ? clamp_magic(c[e] + z, 0.0f, 15.0f) : clamp_magic(c[e], -lim, lim);
         if (in) store8(q + row * ldq + col / 2, nibbles8<FMT == 1>(c), nibbles8<FMT == 1>(c + 8), wide);
         const bool lead = in && (lane & 12) == 0;   // one lane per group, of column col
         if (lead) {

@@ -125,3 +125,24 @@ def test_decode_to_tiles(gpu_device, n, k, gs, shift):
     assert torch.equal(tiles, ops.tile_int8_weight(rows)) and np.array_equal(rs.cpu().numpy(), sc)
     p = ck.PreparedW4A8(q, *args, gs)
     assert (p.n, p.k) == (n, k) and torch.equal(p.q8, tiles) and torch.equal(p.row_scale, rs)
+
+
+@pytest.mark.parametrize("cg", [0, 64, 256])
+def test_nan_in_groups_of_scale_zero(gpu_device, cg):
+    """A group whose scale is 0 (wholly NaN, as one NaN weight makes its whole Hadamard block, or too
+    small for fp16) stores codes and zero-points of 0, NaN weights included."""
+    print(f"[wquant] NaN, scale 0, cg={cg}", flush=True)
+    w = torch.linspace(-1.0, 1.0, 512, device=gpu_device).repeat(3, 1)
+    w[0, 64:128] = float("nan")
+    w[1, 300] = float("nan")
+    w[2, :256] = 1.0e-9
+    w[2, 7] = float("nan")
+    for fn in (weights.quantize_w4a4_group_weight, weights.quantize_w4a8_asym_weight):
+        out = fn(w, 64, cg)
+        q, s = out[0].view(torch.uint8).view(3, 8, 32).cpu(), out[1].float().cpu()
+        zero = s == 0
+        assert zero[0, 1] and zero[2, 0] and (cg == 0 or zero[1].any())
+        assert not q[zero].any() and q[~zero].any()
+        if len(out) == 3:
+            z = torch.stack([out[2].cpu() & 15, out[2].cpu() >> 4], 2).view(3, 8)
+            assert not z[zero].any()
