@@ -85,8 +85,9 @@ def _hip_quantize(weight: torch.Tensor, convrot_groupsize: int | None, fmt: int)
     q = torch.empty((n, k if fmt == _lib.WFMT_I8_ROW else k // 2), dtype=qdt, device=dev)
     s = torch.empty((n, k // 64) if group else (n,), dtype=torch.float16 if group else torch.float32, device=dev)
     z = torch.empty((n, (k // 64 + 1) // 2), dtype=torch.uint8, device=dev) if fmt == _lib.WFMT_U4_ASYM_G64 else None
-    # a group whose range overflows its fp16 scale: the kernel says so in pinned host memory
-    bad = torch.zeros(1, dtype=torch.int32, pin_memory=True) if group else None
+    # a group whose range overflows its fp16 scale: the kernel says so in pinned host memory (whatever the
+    # caller's default device is)
+    bad = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True) if group else None
     _lib.call("mq_quantize_weight_checked", w.data_ptr(), dts[w.dtype], n, k, w.stride(0), cg, fmt, q.data_ptr(),
               q.stride(0), s.data_ptr(), s.stride(0) if group else 1, _lib.ptr(z), z.stride(0) if z is not None else 0,
               _lib.ptr(bad), _lib.stream_of(w))

@@ -146,3 +146,16 @@ def test_nan_in_groups_of_scale_zero(gpu_device, cg):
         if len(out) == 3:
             z = torch.stack([out[2].cpu() & 15, out[2].cpu() >> 4], 2).view(3, 8)
             assert not z[zero].any()
+
+
+def test_group_formats_under_a_default_device(gpu_device):
+    """With a default device set, as loaders that build modules on the GPU do: the overflow flag is host
+    memory whatever the default is."""
+    print("[wquant] default device", flush=True)
+    w = torch.linspace(-1.0, 1.0, 512, device=gpu_device).repeat(3, 1)
+    want = weights.quantize_w4a8_asym_weight(w, 64, 64) + weights.quantize_w4a4_group_weight(w, 64, 64)
+    with torch.device(gpu_device):
+        got = weights.quantize_w4a8_asym_weight(w, 64, 64) + weights.quantize_w4a4_group_weight(w, 64, 64)
+        with pytest.raises(ValueError, match="overflows the fp16 scale"):
+            weights.quantize_w4a4_group_weight(w * 1e7, 64, 64)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
