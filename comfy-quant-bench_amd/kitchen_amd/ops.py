@@ -589,8 +589,8 @@ def _linear_w4_group(x, swiglu, cg, act_bits, qweight, wscales, wzeros, bias, n,
             zz = wzeros.contiguous()
             zptr, ldwz = zz.data_ptr(), zz.shape[1]
     bptr, bdt = (None, _lib.DT_BF16) if b is None else (b.data_ptr(), _lib.DTYPE_CODE[b.dtype])
-    _lib.call("mq_linear_w4_group", x2.data_ptr(), _lib.DTYPE_CODE[x2.dtype], 2 * k if swiglu else k, cg or 0, ab,
-              swiglu, qptr, ldw, wscales.data_ptr(), wscales.stride(0), zptr, ldwz, bptr, bdt, y.data_ptr(),
+    _lib.call("mq_linear_w4_group", x2.data_ptr(), _lib.DTYPE_CODE[x2.dtype], 2 * k if swiglu else k, int(cg or 0),
+              ab, swiglu, qptr, ldw, wscales.data_ptr(), wscales.stride(0), zptr, ldwz, bptr, bdt, y.data_ptr(),
               _lib.DTYPE_CODE[out_dtype], n, m, n, k, work.data_ptr(), work.numel(), stream)
     return y
 
@@ -618,8 +618,8 @@ def _linear_rowscale(x, swiglu, cg, act_bits, qweight, wbits, wscales, bias, n, 
     stream = _lib.stream_of_device(dev)
     work = _linear_workspace(m, n, k, dev, stream)
     bptr, bdt = (None, _lib.DT_BF16) if b is None else (b.data_ptr(), _lib.DTYPE_CODE[b.dtype])
-    _lib.call("mq_linear_rowscale", x2.data_ptr(), _lib.DTYPE_CODE[x2.dtype], 2 * k if swiglu else k, cg or 0, act_bits,
-              swiglu, qw.data_ptr(), ldw, wbits, wscales.data_ptr(), bptr, bdt, y.data_ptr(),
+    _lib.call("mq_linear_rowscale", x2.data_ptr(), _lib.DTYPE_CODE[x2.dtype], 2 * k if swiglu else k, int(cg or 0),
+              act_bits, swiglu, qw.data_ptr(), ldw, wbits, wscales.data_ptr(), bptr, bdt, y.data_ptr(),
               _lib.DTYPE_CODE[out_dtype], n, m, n, k, work.data_ptr(), work.numel(), stream)
     return y
 
