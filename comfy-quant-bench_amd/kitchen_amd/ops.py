@@ -564,6 +564,14 @@ def _linear_input(x: torch.Tensor, swiglu: int, k: int):
     return x2, swiglu
 
 
+def _output(x2: torch.Tensor, m: int, n: int, out_dtype) -> torch.Tensor:
+    """A linear's output [M, N] on x2's device: a plain tensor whatever x2's class (new_empty, which keeps
+    the class, is the cheaper call: one-row linears are bound by their host time)."""
+    if type(x2) is not torch.Tensor:
+        return torch.empty((m, n), dtype=out_dtype, device=x2.device)
+    return x2.new_empty((m, n)) if out_dtype is x2.dtype else x2.new_empty((m, n), dtype=out_dtype)
+
+
 def _linear_w4_group(x, swiglu, cg, act_bits, qweight, wscales, wzeros, bias, n, k, out_dtype):
     """rotate + quantize + group GEMM in one library call (mq_linear_w4_group)."""
     x2, swiglu = _linear_input(x, swiglu, k)
@@ -571,7 +579,7 @@ def _linear_w4_group(x, swiglu, cg, act_bits, qweight, wscales, wzeros, bias, n,
     _check_w4_group_weights(qweight, wscales, wzeros, n, k, INT4_GROUP_SIZE)
     dev = x2.device
     b = _bias(bias, n, dev)
-    y = x2.new_empty((m, n)) if out_dtype is x2.dtype else x2.new_empty((m, n), dtype=out_dtype)
+    y = _output(x2, m, n, out_dtype)
     if m == 0:
         return y
     stream = _lib.stream_of_device(dev)
@@ -612,7 +620,7 @@ def _linear_rowscale(x, swiglu, cg, act_bits, qweight, wbits, wscales, bias, n, 
     ldw, wbits = _weight_args(qw, n, k, wbits) if tiles else (wbytes, wbits)
     dev = x2.device
     b = _bias(bias, n, dev)
-    y = x2.new_empty((m, n)) if out_dtype is x2.dtype else x2.new_empty((m, n), dtype=out_dtype)
+    y = _output(x2, m, n, out_dtype)
     if m == 0:
         return y
     stream = _lib.stream_of_device(dev)

@@ -46,3 +46,14 @@ def test_convrot_groupsize_of_any_number_type(calls, cg):
     ys = _linears(torch.zeros((3, 256), dtype=torch.bfloat16), cg)
     assert [y.shape for y in ys] == [(3, 8)] * 4 and len(calls) == 4
     assert all(args[3] == 256 for _, args in calls)
+
+
+def test_outputs_are_plain_tensors(calls):
+    """The outputs are the library's own buffers, not the class of the activations."""
+    class Tagged(torch.Tensor):
+        pass
+
+    for dtype in (torch.bfloat16, torch.float32):
+        x = torch.zeros((3, 256), dtype=dtype)
+        assert [type(y) for y in _linears(x.as_subclass(Tagged), 256)] == [torch.Tensor] * 4
+        assert [(type(y), y.dtype, y.device) for y in _linears(x, 256)] == [(torch.Tensor, dtype, x.device)] * 4
