@@ -36,6 +36,7 @@ torch on the input's device, and the HIP kernels run asynchronously on the curre
 from __future__ import annotations
 
 import os
+import threading
 import weakref
 
 import torch
@@ -249,21 +250,29 @@ def _check_w4_group_weights(qweight, wscales, wzeros, n, k, group_size):
 _WS_BYTES: dict = {}
 _LINEAR_WS_BYTES: dict = {}
 
-# Workspaces up to this size are kept per (device, stream) and reused by the next call on that
-# stream (calls on one stream run in order, so they never overlap); larger ones, and every
-# workspace taken while a HIP graph is being captured (the graph's own pool then holds it), are
-# allocated per call.
+# Workspaces up to this size are kept per (thread, device, stream) and reused by that thread's next call
+# on that stream; a thread's are given back when it ends. Calls of one thread on one stream run in
+# order, so they never overlap; those of two threads may, their launches interleaved, as an entry
+# point that launches twice is called without the GIL. Larger workspaces, and every workspace taken
+# while a HIP graph is being captured (the graph's own pool then holds it), are allocated per call.
 WORKSPACE_CACHE_BYTES = 64 << 20
-_WS_CACHE: dict = {}
+
+
+class _Workspaces(threading.local):
+    def __init__(self):
+        self.by_stream: dict = {}   # (device index, stream) -> buffer
+
+
+_WORKSPACES = _Workspaces()
 
 
 def _scratch(nbytes: int, device, stream: int) -> torch.Tensor:
     if nbytes > WORKSPACE_CACHE_BYTES or torch.cuda.is_current_stream_capturing():
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
-    key = (device.index, stream)
-    buf = _WS_CACHE.get(key)
+    kept, key = _WORKSPACES.by_stream, (device.index, stream)
+    buf = kept.get(key)
     if buf is None or buf.numel() < nbytes:
-        buf = _WS_CACHE[key] = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        buf = kept[key] = torch.empty(nbytes, dtype=torch.uint8, device=device)
     return buf
 
 

@@ -1,6 +1,8 @@
 """The host side of the linears, on the CPU: what is handed to the library, what comes back, and the
 workspaces that calls share. The library is called with no rows, so nothing is launched."""
+import gc
 import threading
+import weakref
 
 import pytest
 import torch
@@ -57,3 +59,28 @@ def test_outputs_are_plain_tensors(calls):
         x = torch.zeros((3, 256), dtype=dtype)
         assert [type(y) for y in _linears(x.as_subclass(Tagged), 256)] == [torch.Tensor] * 4
         assert [(type(y), y.dtype, y.device) for y in _linears(x, 256)] == [(torch.Tensor, dtype, x.device)] * 4
+
+
+def test_threads_on_one_stream_have_their_own_workspaces(monkeypatch):
+    """A linear launches twice (codes into the workspace, then the product that reads them) and its call
+    releases the GIL: a second thread on the same stream may not be handed the same workspace."""
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    cpu, got, refs = torch.device("cpu"), {}, {}
+    barrier = threading.Barrier(2)
+
+    def work(name):
+        a = ops._scratch(1000, cpu, 7)
+        barrier.wait(10)
+        got[name] = (a.data_ptr(), ops._scratch(900, cpu, 7) is a, ops._scratch(1000, cpu, 8) is a)
+        refs[name] = weakref.ref(a)
+        barrier.wait(10)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(20)
+    assert got[0][0] != got[1][0]
+    assert all(again and not other for _, again, other in got.values())   # kept per stream, in each thread
+    gc.collect()
+    assert refs[0]() is None and refs[1]() is None                        # and given back when it ends
