@@ -95,4 +95,9 @@ static PyMethodDef methods[] = {
 };
 static struct PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fast", NULL, -1, methods, NULL, NULL, NULL, NULL};
 
-PyMODINIT_FUNC PyInit__fast(void) { return PyModule_Create(&module); }
+/* ABI_VERSION: of the header whose argument orders are compiled in above */
+PyMODINIT_FUNC PyInit__fast(void) {
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddIntConstant(m, "ABI_VERSION", MQ_ABI_VERSION) < 0) Py_CLEAR(m);
+    return m;
+}

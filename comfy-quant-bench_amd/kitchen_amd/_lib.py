@@ -111,6 +111,9 @@ def load() -> ctypes.CDLL:
     except ImportError as e:
         raise RuntimeError(f"{os.path.join(_HERE, '_fast.so')} is not built: run `python comfy-quant-bench_amd/build.py` "
                            "(or __graft_entry__.build()) first") from e
+    ver = getattr(_fast, "ABI_VERSION", None)
+    if ver != ABI_VERSION:
+        raise RuntimeError(f"_fast.so was built for ABI version {ver}, expected {ABI_VERSION}: rebuild the library")
     _fast.bind(*(ctypes.cast(getattr(lib, name), c_vp).value for name in FAST_ENTRIES))
     _entries.update({name: getattr(lib, name) for name in _SIGNATURES})
     _entries.update({name: getattr(_fast, name) for name in FAST_ENTRIES})

@@ -31,3 +31,30 @@ def test_none_is_a_null_pointer_and_nothing_else(name, args, rows, bad):
                 getattr(lib, name)(*one)
             with pytest.raises(TypeError, match=f"argument {i + 1} "):
                 _lib._entries[name](*one)
+
+
+def _python(code):
+    env = dict(os.environ, PYTHONPATH=PKG_ROOT)
+    return subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env=env, timeout=300)
+
+
+def test_a_module_of_another_abi_version_is_refused():
+    """The order of an entry's arguments is compiled into the module: one built from an older header is not bound."""
+    res = _python("""
+import sys, types
+from kitchen_amd import _lib
+stale = types.ModuleType("kitchen_amd._fast")
+stale.ABI_VERSION = _lib.ABI_VERSION - 1
+stale.bind = lambda *a: print("bound")
+for name in _lib.FAST_ENTRIES:
+    setattr(stale, name, lambda *a: 0)
+sys.modules["kitchen_amd._fast"] = stale
+import kitchen_amd
+kitchen_amd._fast = stale
+try:
+    _lib.load()
+except RuntimeError as e:
+    print("refused:", e)
+""")
+    assert res.returncode == 0, res.stderr
+    assert "bound" not in res.stdout and "refused: " in res.stdout and "rebuild" in res.stdout
