@@ -67,9 +67,20 @@ def _compile(src: str, build_dir: str, verbose: bool) -> str:
 
 
 def _compile_fast() -> None:
+    """_fast.so. Where a C compiler or Python's headers are missing it is left out, and the package calls
+    the same entry points through ctypes."""
+    include = sysconfig.get_paths()["include"]
     cc = shutil.which("gcc") or shutil.which("cc") or os.path.join(os.path.dirname(hipcc()), "amdclang")
+    missing = None if os.path.exists(cc) else "no C compiler"
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        missing = f"no Python.h in {include}"
+    if missing:
+        print(f"_fast.so is not built: {missing}", file=sys.stderr)
+        if os.path.exists(FAST):
+            os.remove(FAST)
+        return
     tmp = FAST + ".tmp"
-    cmd = [cc, "-O2", "-shared", "-fPIC", "-Wall", "-Wno-unused-function", "-I", sysconfig.get_paths()["include"],
+    cmd = [cc, "-O2", "-shared", "-fPIC", "-Wall", "-Wno-unused-function", "-I", include,
            os.path.join(CSRC, "mq_fast.c"), "-o", tmp]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:

@@ -1,7 +1,8 @@
 """ctypes binding of libmq.so (C ABI in include/mq.h).
 
 The entry points that a linear or an activation quantizer makes per call go through the CPython module
-_fast.so (csrc/mq_fast.c), bound to the same loaded library; all others through ctypes.
+_fast.so (csrc/mq_fast.c), bound to the same loaded library; all others, and those too where that module is
+not built, through ctypes.
 
 The library is loaded after `import torch`, so its `libamdhip64.so.7` dependency resolves to the
 HIP runtime torch already mapped: device pointers, streams and the kernels share one runtime.
@@ -11,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 
 import torch  # noqa: F401  (must be imported before the library is loaded)
 
@@ -106,17 +108,17 @@ def load() -> ctypes.CDLL:
     ver = lib.mq_abi_version()
     if ver != ABI_VERSION:
         raise RuntimeError(f"libmq ABI version {ver}, expected {ABI_VERSION}: rebuild the library")
+    _entries.update({name: getattr(lib, name) for name in _SIGNATURES})
     try:
         from . import _fast
-    except ImportError as e:
-        raise RuntimeError(f"{os.path.join(_HERE, '_fast.so')} is not built: run `python comfy-quant-bench_amd/build.py` "
-                           "(or __graft_entry__.build()) first") from e
-    ver = getattr(_fast, "ABI_VERSION", None)
-    if ver != ABI_VERSION:
-        raise RuntimeError(f"_fast.so was built for ABI version {ver}, expected {ABI_VERSION}: rebuild the library")
-    _fast.bind(*(ctypes.cast(getattr(lib, name), c_vp).value for name in FAST_ENTRIES))
-    _entries.update({name: getattr(lib, name) for name in _SIGNATURES})
-    _entries.update({name: getattr(_fast, name) for name in FAST_ENTRIES})
+    except ImportError as e:   # not built: the same entries through ctypes, a microsecond more each
+        warnings.warn(f"{os.path.join(_HERE, '_fast.so')} cannot be imported ({e}): calls go through ctypes")
+    else:
+        ver = getattr(_fast, "ABI_VERSION", None)
+        if ver != ABI_VERSION:
+            raise RuntimeError(f"_fast.so was built for ABI version {ver}, expected {ABI_VERSION}: rebuild the library")
+        _fast.bind(*(ctypes.cast(getattr(lib, name), c_vp).value for name in FAST_ENTRIES))
+        _entries.update({name: getattr(_fast, name) for name in FAST_ENTRIES})
     _lib = lib
     return lib
 

@@ -58,3 +58,43 @@ except RuntimeError as e:
 """)
     assert res.returncode == 0, res.stderr
     assert "bound" not in res.stdout and "refused: " in res.stdout and "rebuild" in res.stdout
+
+
+def test_without_the_module_the_calls_go_through_ctypes():
+    """Where _fast.so is not built, the same library's entries are called through ctypes, with a warning."""
+    res = _python("""
+import sys, warnings
+sys.modules["kitchen_amd._fast"] = None
+from kitchen_amd import _lib
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    lib = _lib.load()
+assert len(seen) == 1 and "_fast.so" in str(seen[0].message), seen
+for name in _lib.FAST_ENTRIES:
+    assert _lib._entries[name] is getattr(lib, name)
+A = 1 << 20
+_lib.call("mq_rotquant", A, 0, 0, 256, 256, 256, 8, 0, A, 256, A, None)
+try:
+    _lib.call("mq_rotquant", A, 0, 4, 256, 256, 256, 5, 0, A, 256, A, None)
+except ValueError as e:
+    print("refused:", e)
+""")
+    assert res.returncode == 0, res.stderr
+    assert "refused: mq_rotquant" in res.stdout
+
+
+@pytest.mark.parametrize("missing", ["headers", "compiler"])
+def test_build_without_headers_or_compiler(monkeypatch, tmp_path, missing):
+    """The library is built all the same, and no module of an earlier build is left behind."""
+    import build
+
+    fast = tmp_path / "_fast.so"
+    fast.write_bytes(b"old")
+    monkeypatch.setattr(build, "FAST", str(fast))
+    if missing == "headers":
+        monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    else:
+        monkeypatch.setattr(build, "hipcc", lambda: str(tmp_path / "hipcc"))
+        monkeypatch.setattr(build.shutil, "which", lambda name: None)
+    build._compile_fast()
+    assert not fast.exists()
