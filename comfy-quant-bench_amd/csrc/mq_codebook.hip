@@ -15,9 +15,11 @@
 // tiling them in a second pass. A thread makes 16 consecutive k of one row (8 packed bytes in, 16
 // bytes out; one scale where the group is 16 or more), a wavefront one tile, or 1024 columns of a row.
 //
-// What bounds it: HBM, 1.5 bytes per weight and the scales. N = 12288, K = 3072, group 16, to tiles
-// (59 MB): 15.8 us. (One workgroup per row, eight k per thread step with an integer division and a
-// scale byte load per weight, took 47.1 us to rows, and the tiling pass 11.6 more.)
+// What bounds it: HBM, 1.5 bytes per weight and the scales. N = 12288, K = 3072 to tiles (59 MB at group 16),
+// calls back to back: 15.4-15.6 us a call at groups of 16, 32, 48, 64 and 128 (16.4 with an integer
+// division per lane for the group index, GroupIndex below); to rows 16.1-16.4 (17.3). (One workgroup per row,
+// eight k per thread step with an integer division and a scale byte load per weight, took 47.1 us to
+// rows, and the tiling pass 11.6 more.)
 #include <algorithm>
 
 #include "mq_device.h"
@@ -40,12 +42,31 @@ __device__ __forceinline__ float fp8_e4m3fn(uint32_t b) {
     return (b & 0x80u) ? -v : v;
 }
 
+// k / gs for a column k that is a multiple of 16 and a group size of 16 d, without a division (gs is a
+// run-time value, and an integer division a dozen instructions a lane): with u = k / 16 < 2^26,
+// l = ceil(log2 d) and m = ceil(2^(26 + l) / d) = (2^(26 + l) + e) / d, e < d <= 2^l, the excess of
+// u m / 2^(26 + l) over u / d is u e / (d 2^(26 + l)) < 1 / d, so its floor is u / d's. As one high product:
+// (2 u) (32 m) / 2^32 = u m / 2^26, and m < 2^27 keeps 32 m in 32 bits (d < 2^26). The same work for every gs.
+struct GroupIndex {
+    uint32_t mul;
+    int shift;
+    __device__ __forceinline__ uint32_t operator()(int k) const {
+        return __umulhi(static_cast<uint32_t>(k) >> 3, mul) >> shift;
+    }
+};
+GroupIndex group_index(int gs) {
+    const uint64_t d = static_cast<uint64_t>(std::max(gs / 16, 1));   // (groups under 16 are not indexed this way)
+    int l = 0;
+    while ((uint64_t(1) << l) < d) ++l;
+    return {static_cast<uint32_t>(((uint64_t(1) << (26 + l)) + d - 1) / d) << 5, l};
+}
+
 // Units of 64 threads (one wavefront): tile t = band * (K / 64) + g, lane = (row, 16-column chunk); or,
 // to rows, the part'th 1024 columns of a row. SPU: scales per 16 columns (1: group_size >= 16).
 template <bool TILE, int SPU>
 __global__ void __launch_bounds__(64 * kWaves)
 decode_kernel(const uint8_t* __restrict__ qdata, int64_t ldq, const uint8_t* __restrict__ s_rel, int64_t lds,
-              const float* __restrict__ s_channel, const float* __restrict__ codebook, int gs, int64_t N, int K,
+              const float* __restrict__ s_channel, const float* __restrict__ codebook, GroupIndex group, int64_t N, int K,
               int8_t* __restrict__ q8, int64_t ldq8, float* __restrict__ row_scale) {
     __shared__ float lev[16];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -77,7 +98,7 @@ decode_kernel(const uint8_t* __restrict__ qdata, int64_t ldq, const uint8_t* __r
             float s[SPU];
 #pragma unroll
             for (int j = 0; j < SPU; ++j)
-                s[j] = fp8_e4m3fn(s_rel[n * lds + (SPU > 1 ? k / (16 / SPU) + j : gs == 16 ? k >> 4 : k / gs)]);
+                s[j] = fp8_e4m3fn(s_rel[n * lds + (SPU > 1 ? k / (16 / SPU) + j : group(k))]);
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const float t = lev[(w[i >> 3] >> (4 * (i & 7))) & 0xfu] * s[i * SPU / 16];
@@ -106,7 +127,7 @@ int launch_decode_w4a8_codebook(const uint8_t* qdata, int64_t ldq, const uint8_t
     const dim3 grid(static_cast<unsigned>(std::min<int64_t>((units + kWaves - 1) / kWaves, int64_t(1) << 22)));
 #define MQ_DC(TILE, SPU)                                                                                           \
     hipLaunchKernelGGL((decode_kernel<TILE, SPU>), grid, dim3(64 * kWaves), 0, stream, qdata, ldq, s_rel, lds,      \
-                       s_channel, codebook, group_size, N, static_cast<int>(K), q8, ldq8, row_scale)
+                       s_channel, codebook, group_index(group_size), N, static_cast<int>(K), q8, ldq8, row_scale)
     if (group_size >= 16) {
         if (tile) MQ_DC(true, 1);
         else MQ_DC(false, 1);

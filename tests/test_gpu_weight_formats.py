@@ -159,3 +159,19 @@ def test_group_formats_under_a_default_device(gpu_device):
         with pytest.raises(ValueError, match="overflows the fp16 scale"):
             weights.quantize_w4a4_group_weight(w * 1e7, 64, 64)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("n,k,gs", [(17, 960, 48), (5, 1280, 80), (3, 2016, 112), (16, 1024, 1024), (33, 3072, 768)])
+def test_decode_group_sizes(gpu_device, n, k, gs):
+    """Groups that are no power of two, and one group a row: rows and, where K allows, tiles."""
+    print(f"[codebook] group sizes N={n} K={k} gs={gs}", flush=True)
+    rng = np.random.default_rng(gs)
+    qd = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
+    sr, sc = rng.integers(0, 256, (n, k // gs), dtype=np.uint8), rng.uniform(0.001, 0.05, n).astype(np.float32)
+    cb = np.sort(rng.uniform(-1, 1, 16)).astype(np.float32)
+    q0, _ = cbk.decode_w4a8_codebook(qd, sr, sc, cb, gs)
+    args = [torch.from_numpy(a).to(gpu_device) for a in (qd, sr, sc, cb)]
+    q, _ = ops.decode_w4a8_codebook_weight(*args, gs)
+    assert np.array_equal(q.cpu().numpy(), q0)
+    if k % 64 == 0:
+        assert torch.equal(ck.PreparedW4A8(*args, gs).q8, ops.tile_int8_weight(q))
