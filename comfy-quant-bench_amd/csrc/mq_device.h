@@ -78,6 +78,10 @@ constexpr int kQuadPerm0022 = 0xA0;   // lane <- lane & ~1 within the quad
 constexpr int kQuadPerm1133 = 0xF5;   // lane <- lane | 1
 constexpr int kQuadPerm0101 = 0x44;   // lane <- lane & ~2
 constexpr int kQuadPerm2323 = 0xEE;   // lane <- lane | 2
+constexpr int kRowShl4 = 0x104;       // lane <- lane + 4 (within a row of 16)
+constexpr int kRowShl8 = 0x108;
+constexpr int kRowShr4 = 0x114;       // lane <- lane - 4
+constexpr int kRowShr8 = 0x118;
 
 // Maximum over the 64 lanes of a wavefront, returned in every lane: four DPP steps give each
 // 16-lane row its maximum, then the four row maxima are read as scalars (no LDS round trip).

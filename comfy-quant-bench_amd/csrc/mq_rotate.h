@@ -37,7 +37,59 @@ __device__ __forceinline__ void stage_reg(float (&v)[16]) {
     }
 }
 
-// The rotation of a chunk, its lane exchanges done through LDS (no VALU work for them). Within each group of 16 lanes that share lane bits L0 L1, lane bits L2..L5 hold c4..c7
+// Exchange lane bit B (2..5) with register bit J of an array of N 32-bit values: afterwards the
+// value with (lane bit B = u, register bit J = w) is the one that was at (lane bit B = w,
+// register bit J = u).
+template <int B, int J, int N, typename T>
+__device__ __forceinline__ void swap_lane_reg(T (&v)[N], [[maybe_unused]] int lane) {
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+        if (r & (1 << J)) continue;
+        const uint32_t x = __builtin_bit_cast(uint32_t, v[r]), y = __builtin_bit_cast(uint32_t, v[r | (1 << J)]);
+        uint32_t xn, yn;
+        if constexpr (B == 2 || B == 3) {
+            // lanes with the bit set take y from lane - 2^B, the others x from lane + 2^B: row
+            // shifts within 16-lane rows, each written only into the lanes (DPP banks of 4 lanes =
+            // lane bits 2, 3) that take it, so every moved value costs one v_mov_b32_dpp
+            constexpr int shr = B == 2 ? kRowShr4 : kRowShr8, shl = B == 2 ? kRowShl4 : kRowShl8;
+            constexpr int up = B == 2 ? 0xA : 0xC;        // banks with the lane bit set
+            xn = __builtin_amdgcn_update_dpp(x, y, shr, 0xf, up, false);
+            yn = __builtin_amdgcn_update_dpp(y, x, shl, 0xf, up ^ 0xf, false);
+        } else if constexpr (B == 4) {
+            const auto p = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+            xn = p[0];
+            yn = p[1];
+        } else {
+            static_assert(B == 5, "lane bit");
+            const auto p = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+            xn = p[0];
+            yn = p[1];
+        }
+        v[r] = __builtin_bit_cast(T, xn);
+        v[r | (1 << J)] = __builtin_bit_cast(T, yn);
+    }
+}
+
+template <int BLK>
+__device__ __forceinline__ void rotate_chunk(float (&v)[16], int lane) {
+    if constexpr (BLK >= 16) {
+        stage_reg<0>(v);          // element stride 1  (c0 c1)
+        stage_reg<2>(v);          // element stride 4  (c2 c3)
+    }
+    if constexpr (BLK >= 64) {
+        swap_lane_reg<2, 2>(v, lane);
+        swap_lane_reg<3, 3>(v, lane);
+        stage_reg<2>(v);          // element stride 16 (c4 c5)
+    }
+    if constexpr (BLK >= 256) {
+        swap_lane_reg<4, 2>(v, lane);
+        swap_lane_reg<5, 3>(v, lane);
+        stage_reg<2>(v);          // element stride 64 (c6 c7)
+    }
+}
+
+// The same rotation with the exchanges done through LDS instead of lane swaps (no VALU work for them) and
+// back in the load layout. Within each group of 16 lanes that share lane bits L0 L1, lane bits L2..L5 hold c4..c7
 // and the 16 registers c0..c3: a 16 x 16 transpose (lane index <-> register index) brings c4..c7
 // into the registers, where the stages over (c4 c5) and (c6 c7) run, and the same transpose
 // brings the load layout back. Lane (g, i) = (L & 3, L >> 2) writes its register j at float
@@ -106,6 +158,13 @@ __device__ __forceinline__ float recip_row(float s) {
     const float e = __builtin_fmaf(-s, r0, 1.0f);
     const float r = __builtin_fmaf(e, r0, r0);
     return s == __builtin_inff() ? 0.0f : r;
+}
+
+// Column bit 6 (the parity of the 64-column group) of register r of lane L after rotate_chunk.
+template <int BLK>
+__device__ __forceinline__ int col_bit6(int lane, int r) {
+    if constexpr (BLK >= 256) return (r >> 2) & 1;   // r2 r3 hold c6 c7
+    else return (lane >> 4) & 1;                      // L4 holds c6
 }
 
 // Quantize 16 values: fast path for all, then (rarely, per lane) the exact path for the values

@@ -20,7 +20,13 @@
 // stages over (c4 c5) and (c6 c7) run there and the same transpose brings the load layout back, so the
 // exchanges cost no VALU instructions, every butterfly runs in registers in the reference's order, and
 // a lane's four dwords of codes are 16 consecutive columns, written with one 16-byte (int8) or 8-byte
-// (packed int4) store.
+// (packed int4) store. The fp16 SwiGLU kernels exchange through lanes instead (rotate_chunk: DPP row shifts and
+// v_permlane16 / 32_swap), which leaves c6 c7 (block 256) or c4 c5 (block 64) in r2 r3, and turn the
+// layout back on the dwords of codes. They wait for gathers from a 256 KB table in global memory, for which
+// VALU instructions cost nothing, and with the LDS transpose they were slower: us, lane swaps / LDS, packed
+// int4: 32760 x 3072 213 / 264, 4096 x 9216 77 / 85, 4096 x 5120 43.6 / 48.4, 4096 x 12288 98 / 103 (its
+// smaller register need lets more waves on a unit, whose gathers push each other out of the L1: with the
+// occupancy held down by unused LDS it gave 216, 81, 44.8 and 97).
 //
 // Quantization without a per-element division: with r within 2^-23 relative of 1/s,
 // m = fma(v, r, 1.5*2^23) rounds v*r to an integer n. |v*r - v/s| < 2^-16 and
@@ -195,12 +201,16 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
                 uint8_t* __restrict__ q, int64_t ldq, float* __restrict__ scale, bool nt) {
     constexpr int LIMIT = OUT == 0 ? 127 : 7;
     constexpr int RPG = kWaves / W;                      // rows per workgroup step
+    // how lanes and registers are exchanged (the fp16 SwiGLU kernels: through lanes), and the block whose
+    // register layout the rotated values are in (16: the load layout)
+    constexpr bool kLdsT = BLK >= 64 && !(ACT >= 1 && IN == 1);
+    constexpr int LB = kLdsT ? 16 : BLK;
     const int lane = threadIdx.x & 63;
     int wave = threadIdx.x >> 6;
     if constexpr (DEAD) wave = __builtin_amdgcn_readfirstlane(wave);
     const int wr = wave % W;                             // this wave's share of its row
     [[maybe_unused]] LdsTranspose tr{nullptr, nullptr};
-    if constexpr (BLK >= 64) {
+    if constexpr (kLdsT) {
         __shared__ __attribute__((aligned(16))) float tr_lds[kWaves * kTrWave];
         float* base = tr_lds + wave * kTrWave + (lane & 3) * kTrG;
         tr.w = base + (lane >> 2);
@@ -221,7 +231,9 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
         __shared__ float red_lds[2][kWaves];
         red = &red_lds[0][0];
     }
-    const int seg = (lane >> 2) + 16 * (lane & 3);   // 16-column segment this lane loads, rotates and stores
+    const int seg = (lane >> 2) + 16 * (lane & 3);   // 16-column segment this lane loads
+    // and the one whose 16 codes it holds in the end
+    const int seg_st = LB >= 256 ? (lane >> 4) + 4 * ((lane >> 2) & 3) + 16 * (lane & 3) : seg;
     [[maybe_unused]] bool last = true;                   // whether this wave's last chunk lies in the row
     if constexpr (DEAD) last = ((NCH - 1) * W + wr) * 1024 < K;
     const int64_t groups = (static_cast<int64_t>(M) + RPG - 1) / RPG;
@@ -301,7 +313,8 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
             if (DEAD && c == NCH - 1 && !last) break;
-            rotate_chunk_lds<BLK>(v[c], tr);
+            if constexpr (kLdsT) rotate_chunk_lds<BLK>(v[c], tr);
+            else rotate_chunk<BLK>(v[c], lane);
             float amc = 0.0f;
 #pragma unroll
             for (int j = 0; j < 16; ++j) amc = __builtin_fmaxf(amc, __builtin_fabsf(v[c][j]));
@@ -329,14 +342,20 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
         for (int c = 0; c < NCH; ++c) {
             if (DEAD && c == NCH - 1 && !last) break;
             // quantization is odd-symmetric (rint and the clamp are), so negating the input of an
-            // odd 64-column group (column bit 6 is lane bit 4) negates its codes exactly
+            // odd 64-column group negates its codes exactly; in block 256's lane-swap layout the group's
+            // parity is register bit r2, so the sign applies per dword below instead
             float mq[16];
-            quant16<LIMIT>(v[c], OUT == 3 && ((lane >> 4) & 1) ? -1.0f : 1.0f, r, s, mq);
+            quant16<LIMIT>(v[c], OUT == 3 && LB < 256 && col_bit6<LB>(lane, 0) ? -1.0f : 1.0f, r, s, mq);
             uint32_t word[4];
 #pragma unroll
             for (int hi = 0; hi < 4; ++hi) {
                 uint32_t m0 = __float_as_uint(mq[4 * hi + 0]), m1 = __float_as_uint(mq[4 * hi + 1]);
                 uint32_t m2 = __float_as_uint(mq[4 * hi + 2]), m3 = __float_as_uint(mq[4 * hi + 3]);
+                if constexpr (OUT == 3 && LB >= 256) {
+                    if (col_bit6<LB>(lane, 4 * hi)) {   // negate the four codes (two's complement bytes)
+                        m0 = -m0; m1 = -m1; m2 = -m2; m3 = -m3;
+                    }
+                }
                 if constexpr (OUT == 3) {
                     m0 <<= 4; m1 <<= 4; m2 <<= 4; m3 <<= 4;
                 }
@@ -348,7 +367,13 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
                     word[hi] = lo16 | hi16;
                 }
             }
-            const int col = (c * W + wr) * 1024 + seg * 16;
+            // dword index bits hold (c6 c7) for block 256 and (c4 c5) for block 64; lane bits L2 L3 hold
+            // (c2 c3): exchanged, each lane's four dwords are consecutive columns
+            if constexpr (LB >= 64) {
+                swap_lane_reg<2, 0>(word, lane);
+                swap_lane_reg<3, 1>(word, lane);
+            }
+            const int col = (c * W + wr) * 1024 + seg_st * 16;
             if (col >= K) continue;
             if constexpr (OUT == 2)
                 store_codes(nt, qr + col / 2, word[0] | (word[1] << 16), word[2] | (word[3] << 16));
@@ -387,16 +412,17 @@ int launch_rq(const uint16_t* x, int64_t M, int64_t K, int64_t ldx, void* q, int
     }
     if (wgs == 0) return 0;
     const bool nt = (OUT == 2 ? M * K / 2 : M * K) >= kNtCodeBytes;
-    const bool dead = W > 1 && K <= (NCH * W - 1) * 1024;
+    constexpr bool kDead = W > 1 && !(ACT >= 1 && IN == 1);   // (nothing is gained where the gathers set the time)
+    const bool dead = kDead && K <= (NCH * W - 1) * 1024;
     // a row stride of 0 asks for the codes in 16-row tiles (one code per byte)
     const bool tiled = OUT != 2 && ldq == 0;
 #define MQ_RQ(TL, DEAD)                                                                                             \
     hipLaunchKernelGGL((rotquant_kernel<BLK, OUT, NCH, ACT, W, IN, TL, DEAD>), dim3(static_cast<unsigned>(wgs)),     \
                        dim3(64 * kWaves), 0, stream, x, ldx, static_cast<int>(M), static_cast<int>(K),              \
                        static_cast<uint8_t*>(q), ldq, scale, nt)
-    if (tiled && dead) MQ_RQ(OUT != 2, (W > 1));
+    if (tiled && dead) MQ_RQ(OUT != 2, kDead);
     else if (tiled) MQ_RQ(OUT != 2, false);
-    else if (dead) MQ_RQ(false, (W > 1));
+    else if (dead) MQ_RQ(false, kDead);
     else MQ_RQ(false, false);
 #undef MQ_RQ
     return launch_status("rotquant");
