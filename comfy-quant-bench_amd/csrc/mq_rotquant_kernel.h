@@ -91,14 +91,10 @@ __device__ __forceinline__ void store_codes(bool nt, uint8_t* p, uint32_t w0, ui
 template <int IN>
 struct SiluF16Table;
 
-// The table's signs are interleaved: entry 2 j + sign for |bits| = kSiluLo + j.
-__device__ __forceinline__ float silu_f32(uint32_t b, float g, const float* tab) {
-    const uint32_t t = b & 0x7fffu;
-    const uint32_t j = __builtin_elementwise_min(t - kSiluLo, kSiluEntries - 1u);   // in bounds always
-    const uint32_t s = __float_as_uint(tab[2 * j + (b >> 15)]);
-    const uint32_t big = (b >> 15) ? 0x80000000u : __float_as_uint(g);
-    const uint32_t r = t < kSiluLo ? __float_as_uint(g * 0.5f) : s;
-    return __uint_as_float(t >= kSiluLo + kSiluEntries ? big : r);
+// silu of a gate (bf16 bits b) outside the table: g / 2 below it, g or -0 from 128 up.
+__device__ __forceinline__ float silu_outside(uint32_t b) {
+    const float g = __uint_as_float(b << 16);
+    return __builtin_fabsf(g) < 1.0f ? g * 0.5f : (b >> 15) ? -0.0f : g;
 }
 
 // The activation of one pair from silu of its gates (s0, s1) and the dword of its ups (two bf16 each), as
@@ -124,17 +120,23 @@ __device__ __forceinline__ void swiglu_product(float s0, float s1, uint32_t wu, 
 // looked up, two at a time in 16-bit halves: y = bits - kSiluLo holds the sign in bit 15 and, in range, j
 // in bits 0 - 11 and zeros in bits 12 - 14 (outside it, some of those are set: kSiluLo is 0x3300 and the
 // table ends at 0x4300), and 8 j + 4 sign, masked into the table whatever y is, is the entry's byte.
-// `out` gathers the y; a lane that finds kSiluOut bits in it forms its values again with silu_f32's closed
-// forms (once for all its chunks, so that their lookups overlap). 7 VALU instructions an element
-// instead of 16, in kernels that the VALU sets; with the rotation's exchanges through LDS instead of
-// lane swaps (4 more): M = 4096, K = 12288, packed int4 59.4 -> 51.1 us (226 MB); M = 32760, K = 3072, int8
-// 126 -> 106 us. (Few long rows gain nothing: M = 16, K = 12288 7.9 -> 8.1 us, latency.)
+// The table's signs are interleaved. `out` gathers the y; a lane that finds kSiluOut bits in it takes the closed
+// form for those gates (0, as all of a padded token's are, or 128 and more, as one channel of a model may
+// be), before the product, from the registers. 7 VALU instructions an element instead of 16, in kernels
+// that the VALU sets; with the rotation's exchanges through LDS instead of lane swaps (4 more), us, packed
+// int4: 4096 x 12288 52.6 -> 42.5, 4096 x 14336 66.5 -> 50.0, 4096 x 4096 24.4 -> 18.1, 32760 x 3072 114 -> 95; with
+// every gate 0 51.7 -> 46.5, 65.1 -> 57.7, 23.7 -> 19.5 and 112 -> 98; with one of a thousand 0 52.6 -> 46.5,
+// 66.7 -> 55.6, 24.5 -> 19.6 and 115 -> 98. (Forming such a lane's values again after all its lookups, from gates and
+// ups loaded a second time, cost 56, 79, 27 and 110 with every gate 0, and the registers for it
+// a third of the waves from 4 chunks up; a branch per pair is better on scattered zeros by 3 %, and worse on
+// whole zero rows by 5 %.)
 constexpr uint32_t kSiluOut = 0x70007000u;
 template <bool EAGER>
-__device__ __forceinline__ void swiglu_lookup(const uint32_t (&w)[8], const uint32_t (&wu)[8], const float* tab,
-                                              float (&v)[16], uint32_t& out) {
+__device__ __forceinline__ void swiglu16(const uint32_t (&w)[8], const uint32_t (&wu)[8], const float* tab, float (&v)[16]) {
     typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
     static_assert(kSiluLo == 0x3300u && kSiluEntries == 4096u, "the range test's bits");
+    float s[16];
+    uint32_t out = 0u;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const u16x2 y = __builtin_bit_cast(u16x2, w[j]) - static_cast<uint16_t>(kSiluLo);
@@ -142,18 +144,21 @@ __device__ __forceinline__ void swiglu_lookup(const uint32_t (&w)[8], const uint
         const uint32_t at = (__builtin_bit_cast(uint32_t, static_cast<u16x2>(y << 3)) & 0x7ff87ff8u) |
                             (__builtin_bit_cast(uint32_t, static_cast<u16x2>(y >> 13)) & 0x00040004u);
         const char* t = reinterpret_cast<const char*>(tab);
-        const float s0 = *reinterpret_cast<const float*>(t + (at & 0xffffu));
-        const float s1 = *reinterpret_cast<const float*>(t + (at >> 16));
-        swiglu_product<EAGER>(s0, s1, wu[j], v[2 * j], v[2 * j + 1]);
+        s[2 * j] = *reinterpret_cast<const float*>(t + (at & 0xffffu));
+        s[2 * j + 1] = *reinterpret_cast<const float*>(t + (at >> 16));
     }
-}
-template <bool EAGER>
-__device__ __forceinline__ void swiglu_any(const uint32_t (&w)[8], const uint32_t (&wu)[8], const float* tab,
-                                           float (&v)[16]) {
+    if (out & kSiluOut) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-        swiglu_product<EAGER>(silu_f32(w[j] & 0xffffu, bf16lo(w[j]), tab), silu_f32(w[j] >> 16, bf16hi(w[j]), tab), wu[j],
-                              v[2 * j], v[2 * j + 1]);
+        for (int j = 0; j < 8; ++j) {
+            const u16x2 y = __builtin_bit_cast(u16x2, w[j]) - static_cast<uint16_t>(kSiluLo);
+            const uint32_t f = __builtin_bit_cast(uint32_t, y) & kSiluOut;
+            const float s0 = silu_outside(w[j] & 0xffffu), s1 = silu_outside(w[j] >> 16);
+            s[2 * j] = f & 0xffffu ? s0 : s[2 * j];
+            s[2 * j + 1] = f >> 16 ? s1 : s[2 * j + 1];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) swiglu_product<EAGER>(s[2 * j], s[2 * j + 1], wu[j], v[2 * j], v[2 * j + 1]);
 }
 
 // fp16 inputs: silu of both gates from the global fp16 table, the products rounded to fp16 (EAGER:
@@ -257,7 +262,7 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
 
         float v[NCH][16];
         bool in[NCH];
-        [[maybe_unused]] uint32_t silu_out = 0u;
+        [[maybe_unused]] uint32_t w[NCH][8], wu[NCH][8];   // 16-bit inputs (gates) and ups, two per dword
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
             const int e0 = (c * W + wr) * 1024 + seg * 16;
@@ -275,38 +280,26 @@ rotquant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
                 }
                 continue;
             }
-            uint32_t w[8];
-            load16bits(xr + e, w);
+            load16bits(xr + e, w[c]);
             if constexpr (ACT >= 1) {
-                uint32_t wu[8];
-                load16bits(xr + K + e, wu);
+                load16bits(xr + K + e, wu[c]);
                 if constexpr (IN == 1) {
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
-                        swiglu_pair_f16<ACT == 2>(w[j], wu[j], tab16, v[c][2 * j], v[c][2 * j + 1]);
-                } else {
-                    swiglu_lookup<ACT == 2>(w, wu, tab, v[c], silu_out);
-                }
+                        swiglu_pair_f16<ACT == 2>(w[c][j], wu[c][j], tab16, v[c][2 * j], v[c][2 * j + 1]);
+                }   // (bf16: formed below, with every chunk's loads issued)
             } else {
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    v[c][2 * j] = IN == 1 ? f16lo(w[j]) : bf16lo(w[j]);
-                    v[c][2 * j + 1] = IN == 1 ? f16hi(w[j]) : bf16hi(w[j]);
+                    v[c][2 * j] = IN == 1 ? f16lo(w[c][j]) : bf16lo(w[c][j]);
+                    v[c][2 * j + 1] = IN == 1 ? f16hi(w[c][j]) : bf16hi(w[c][j]);
                 }
             }
         }
 
         if constexpr (ACT >= 1 && IN == 0) {
-            if (silu_out & kSiluOut) {   // a gate outside the table: the lane's values again, in full
 #pragma unroll
-                for (int c = 0; c < NCH; ++c) {
-                    const int e = in[c] ? (c * W + wr) * 1024 + seg * 16 : 0;
-                    uint32_t w[8], wu[8];
-                    load16bits(xr + e, w);
-                    load16bits(xr + K + e, wu);
-                    swiglu_any<ACT == 2>(w, wu, tab, v[c]);
-                }
-            }
+            for (int c = 0; c < NCH; ++c) swiglu16<ACT == 2>(w[c], wu[c], tab, v[c]);
         }
 
         float am = 0.0f;
