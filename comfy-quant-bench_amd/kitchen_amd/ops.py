@@ -438,10 +438,35 @@ FEW_ROWS = 128
 _EXPANDED: dict = {}
 
 
-def _expansion(qweight, wzeros, layout: int, m: int, k: int, wscales=None):
+class _Ready:
+    """Cached tensors that one stream's kernels write, for calls on any stream: another stream's first use
+    waits for them, and they are not given back before its work with them is done. (Nothing is done
+    under HIP graph capture, which may not wait for work outside the graph: what a captured call reads
+    was made, and waited for, before the capture began.)"""
+
+    __slots__ = ("tensors", "event", "streams")
+
+    def __init__(self, tensors, device, stream: int):
+        self.tensors, self.streams = tensors, {stream}
+        self.event = torch.cuda.Event()
+        self.event.record(torch.cuda.current_stream(device))
+
+    def on(self, device, stream: int) -> None:
+        """Before a launch on `stream`, torch's current stream on `device`."""
+        if stream in self.streams or torch.cuda.is_current_stream_capturing():
+            return
+        current = torch.cuda.current_stream(device)
+        current.wait_event(self.event)
+        for t in self.tensors:
+            t.record_stream(current)
+        self.streams.add(stream)
+
+
+def _expansion(qweight, wzeros, layout: int, m: int, k: int, wscales=None, stream: int = 0):
     """The cached ExpandedW4 of qweight for `layout` when a product of m rows reads one (the wide
     kernel's conditions: K >= 192, K groups in pairs for the group scales' loads, under 2 GiB;
-    the group layouts also carry wscales, fp16 with unit column stride), else None."""
+    the group layouts also carry wscales, fp16 with unit column stride), else None. `stream`: the stream
+    that the product will run on, torch's current one on the weight's device."""
     n = qweight.shape[0]
     if not EXPAND_W4 or m <= (GEMV_ROWS if layout == _lib.W4X_ROW else FEW_ROWS) or k < 192 or k % 64 \
             or _lib.load().mq_expanded_w4_bytes(n, k, int(layout)) >= 1 << 31 or (m + 15) // 16 * 16 * k >= 1 << 31:
@@ -461,6 +486,7 @@ def _expansion(qweight, wzeros, layout: int, m: int, k: int, wscales=None):
     per = _EXPANDED.get(id(root))
     hit = None if per is None else per.get(key)
     if hit is not None and hit[0] == sig:
+        hit[2].on(qweight.device, stream)
         return hit[1]
     if torch.cuda.is_current_stream_capturing():
         return None   # nothing is allocated under capture: the packed weights, unless expanded before
@@ -468,7 +494,7 @@ def _expansion(qweight, wzeros, layout: int, m: int, k: int, wscales=None):
         per = _EXPANDED[id(root)] = {}
         weakref.finalize(root, _EXPANDED.pop, id(root), None)
     ex = expand_w4_weight(qweight, wzeros, layout, None if layout == _lib.W4X_ROW else wscales)
-    per[key] = (sig, ex)
+    per[key] = (sig, ex, _Ready((ex.buf,), qweight.device, stream))
     return ex
 
 
@@ -594,7 +620,7 @@ def _linear_w4_group(x, swiglu, cg, act_bits, qweight, wscales, wzeros, bias, n,
     stream = _lib.stream_of_device(dev)
     work = _linear_workspace(m, n, k, dev, stream)
     xw = None if m <= FEW_ROWS else \
-        _expansion(qweight, wzeros, _lib.ACT_X16ALT if act_bits == 4 else _lib.ACT_I8, m, k, wscales)
+        _expansion(qweight, wzeros, _lib.ACT_X16ALT if act_bits == 4 else _lib.ACT_I8, m, k, wscales, stream)
     if xw is not None:
         qptr, ldw, ab = xw.tiles.data_ptr(), k, act_bits | _lib.W4_EXPANDED
         zptr, ldwz = (xw.tiles.data_ptr() if xw.asym else None), 0   # non-null: uint4 (not read)
@@ -619,20 +645,20 @@ def _linear_rowscale(x, swiglu, cg, act_bits, qweight, wbits, wscales, bias, n, 
     tiles = is_tile16(qweight)
     qw = qweight if tiles else qweight.contiguous()
     wbytes = k // 2 if wbits == 4 else k
+    dev = x2.device
+    stream = _lib.stream_of_device(dev)
     if not tiles and (qw.shape != (n, wbytes) or qw.element_size() != 1):
         raise ValueError(f"weight must be 8-bit [{n}, {wbytes}]")
     if wbits == 4 and m > GEMV_ROWS:
         # signed int4 rows: their int8 expansion where the wide kernel reads it (same int32 sums)
-        xw = _expansion(qweight, None, _lib.W4X_ROW, m, k)
+        xw = _expansion(qweight, None, _lib.W4X_ROW, m, k, stream=stream)
         if xw is not None:
             qw, wbits, tiles = xw.tiles, 8, True
     ldw, wbits = _weight_args(qw, n, k, wbits) if tiles else (wbytes, wbits)
-    dev = x2.device
     b = _bias(bias, n, dev)
     y = _output(x2, m, n, out_dtype)
     if m == 0:
         return y
-    stream = _lib.stream_of_device(dev)
     work = _linear_workspace(m, n, k, dev, stream)
     bptr, bdt = (None, _lib.DT_BF16) if b is None else (b.data_ptr(), _lib.DTYPE_CODE[b.dtype])
     _lib.call("mq_linear_rowscale", x2.data_ptr(), _lib.DTYPE_CODE[x2.dtype], 2 * k if swiglu else k, int(cg or 0),
@@ -654,11 +680,12 @@ def _decoded_w4a8(qdata, s_rel, s_channel, codebook, group_size):
     qid = id(qdata)
     hit = _DECODED.get(qid)
     if hit is not None and hit[0] == sig:
+        hit[2].on(qdata.device, _lib.stream_of(qdata))
         return hit[1]
     dec = decode_w4a8_codebook_weight(qdata, s_rel, s_channel, codebook, group_size)
     if hit is None:
         weakref.finalize(qdata, _DECODED.pop, qid, None)
-    _DECODED[qid] = (sig, dec)
+    _DECODED[qid] = (sig, dec, _Ready(dec, qdata.device, _lib.stream_of(qdata)))
     return dec
 
 
