@@ -440,25 +440,23 @@ _EXPANDED: dict = {}
 
 class _Ready:
     """Cached tensors that one stream's kernels write, for calls on any stream: another stream's first use
-    waits for them, and they are not given back before its work with them is done. (Nothing is done
-    under HIP graph capture, which may not wait for work outside the graph: what a captured call reads
-    was made, and waited for, before the capture began.)"""
+    waits for them on the host, and they are not given back before its work with them is done. (An event
+    behind the making would spare that wait, but costs every weight's first call 8-20 us, two streams or
+    not; recording one later would need the making stream, which may be gone. Nothing is done
+    under HIP graph capture, which may not wait: what a captured call reads was made before it began.)"""
 
-    __slots__ = ("tensors", "event", "streams")
+    __slots__ = ("tensors", "streams")
 
-    def __init__(self, tensors, device, stream: int):
+    def __init__(self, tensors, stream: int):
         self.tensors, self.streams = tensors, {stream}
-        self.event = torch.cuda.Event()
-        self.event.record(torch.cuda.current_stream(device))
 
     def on(self, device, stream: int) -> None:
         """Before a launch on `stream`, torch's current stream on `device`."""
         if stream in self.streams or torch.cuda.is_current_stream_capturing():
             return
-        current = torch.cuda.current_stream(device)
-        current.wait_event(self.event)
+        torch.cuda.synchronize(device)
         for t in self.tensors:
-            t.record_stream(current)
+            t.record_stream(torch.cuda.current_stream(device))
         self.streams.add(stream)
 
 
@@ -494,7 +492,7 @@ def _expansion(qweight, wzeros, layout: int, m: int, k: int, wscales=None, strea
         per = _EXPANDED[id(root)] = {}
         weakref.finalize(root, _EXPANDED.pop, id(root), None)
     ex = expand_w4_weight(qweight, wzeros, layout, None if layout == _lib.W4X_ROW else wscales)
-    per[key] = (sig, ex, _Ready((ex.buf,), qweight.device, stream))
+    per[key] = (sig, ex, _Ready((ex.buf,), stream))
     return ex
 
 
@@ -685,7 +683,7 @@ def _decoded_w4a8(qdata, s_rel, s_channel, codebook, group_size):
     dec = decode_w4a8_codebook_weight(qdata, s_rel, s_channel, codebook, group_size)
     if hit is None:
         weakref.finalize(qdata, _DECODED.pop, qid, None)
-    _DECODED[qid] = (sig, dec, _Ready(dec, qdata.device, _lib.stream_of(qdata)))
+    _DECODED[qid] = (sig, dec, _Ready(dec, _lib.stream_of(qdata)))
     return dec
 
 

@@ -9,19 +9,6 @@ import torch
 from kitchen_amd import _lib, ops
 
 
-class _Stream:
-    def __init__(self):
-        self.waited = []
-
-    def wait_event(self, event):
-        self.waited.append(event)
-
-
-class _Event:
-    def record(self, stream):
-        self.stream = stream
-
-
 class _Buffer:
     def __init__(self):
         self.recorded = []
@@ -32,28 +19,25 @@ class _Buffer:
 
 @pytest.fixture
 def streams(monkeypatch):
-    """Streams 1 and 2; state["now"] is the current one."""
-    state = {"now": 1, "capturing": False, 1: _Stream(), 2: _Stream()}
-    monkeypatch.setattr(torch.cuda, "Event", _Event)
-    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: state[state["now"]])
+    """Streams 1 and 2: state["now"] is the current one, state["waits"] the streams that waited for the device."""
+    state = {"now": 1, "capturing": False, "waits": []}
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda device=None: state["waits"].append(state["now"]))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: state["now"])
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state["capturing"])
     monkeypatch.setattr(_lib, "stream_of_device", lambda device: state["now"])
     return state
 
 
-def _check(state, call, buffers, capture=True):
+def _check(state, call, buffers):
     made = call()
-    assert call() is made and not state[1].waited and not any(b.recorded for b in buffers)
-    state["now"] = 2
-    if capture:   # a capture neither waits nor counts as the stream's first use
-        state["capturing"] = True
-        assert call() is made and not state[2].waited
-        state["capturing"] = False
+    assert call() is made and not any(b.recorded for b in buffers)
+    state["now"], state["capturing"] = 2, True   # a capture neither waits nor counts as the stream's first use
+    assert call() is made and not state["waits"]
+    state["capturing"] = False
     assert call() is made and call() is made
-    assert len(state[2].waited) == 1 and state[2].waited[0].stream is state[1]
-    assert all(b.recorded == [state[2]] for b in buffers)
+    assert state["waits"] == [2] and all(b.recorded == [2] for b in buffers)
     state["now"] = 1
-    assert call() is made and not state[1].waited
+    assert call() is made and state["waits"] == [2]
 
 
 @pytest.mark.parametrize("layout,m", [(_lib.ACT_I8, 200), (_lib.W4X_ROW, 5)])
