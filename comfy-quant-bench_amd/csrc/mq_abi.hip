@@ -498,8 +498,9 @@ struct LinearWs {
 LinearWs linear_ws(int64_t M, int64_t N, int64_t K) {
     LinearWs w;
     w.codes = 0;
-    // codes for M rows rounded up to 16: in the 16-row tile layout the last band spans 16 rows
-    // whatever M is (its rows past M are never written or read)
+    // codes for M rows rounded up to 16: in the 16-row tile layout the last band spans 16 rows whatever
+    // M is. Its rows past M are never written, but the few-row kernel reads them (their products are
+    // dropped at the store), so all 16 have to be there
     w.scales = align_up((M + 15) / 16 * 16 * K);
     w.split = w.scales + align_up(M * 4);
     w.need = w.split;

@@ -83,25 +83,11 @@ constexpr int kRowShl8 = 0x108;
 constexpr int kRowShr4 = 0x114;       // lane <- lane - 4
 constexpr int kRowShr8 = 0x118;
 
-// Maximum over the 64 lanes of a wavefront, returned in every lane: four DPP steps give each
-// 16-lane row its maximum, then the four row maxima are read as scalars (no LDS round trip).
-__device__ __forceinline__ float wave_max(float v) {
-    v = __builtin_fmaxf(v, dpp_mov<kQuadXor1>(v));
-    v = __builtin_fmaxf(v, dpp_mov<kQuadXor2>(v));
-    v = __builtin_fmaxf(v, dpp_mov<kRowRor4>(v));
-    v = __builtin_fmaxf(v, dpp_mov<kRowRor8>(v));
-    const int b = __float_as_int(v);
-    const float r0 = __int_as_float(__builtin_amdgcn_readlane(b, 0));
-    const float r1 = __int_as_float(__builtin_amdgcn_readlane(b, 16));
-    const float r2 = __int_as_float(__builtin_amdgcn_readlane(b, 32));
-    const float r3 = __int_as_float(__builtin_amdgcn_readlane(b, 48));
-    return __builtin_fmaxf(__builtin_fmaxf(r0, r1), __builtin_fmaxf(r2, r3));
-}
-
-// wave_max for values that are >= 0 and not NaN (+inf allowed): their bit patterns order as
-// unsigned integers, so every step is an integer maximum, which takes its DPP operand directly
-// (one instruction per step) and needs none of the float maximum's NaN handling; the four row
-// maxima are combined on the scalar unit.
+// Maximum over the 64 lanes of a wavefront, returned in every lane, of values that are >= 0 and not NaN
+// (+inf allowed): four DPP steps give each 16-lane row its maximum, then the four row maxima are read and
+// combined on the scalar unit (no LDS round trip). The values' bit patterns order as unsigned
+// integers, so every step is an integer maximum, which takes its DPP operand directly (one
+// instruction per step) and needs none of the float maximum's NaN handling.
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_mov_u(uint32_t src) {
     return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(src), CTRL, 0xf, 0xf, true));

@@ -279,7 +279,8 @@ bool gemm_runs_few(const GemmArgs& a, WKind wk, Epi epi) {
     // 32-bit lane offsets over 64 weight rows and 128 activation rows
     constexpr int64_t kMaxStride = int64_t(1) << 23;
     if (a.lda > kMaxStride || a.ldw > kMaxStride || a.ldws > kMaxStride || a.ldwz > kMaxStride) return false;
-    if (epi == Epi::GroupScale) return wk != WKind::I8 && !a.wtile;   // (expanded weights: the wide kernel's)
+    // (expanded weights: the wide kernel's, which is not measured against this one at these rows)
+    if (epi == Epi::GroupScale) return wk != WKind::I8 && !a.wtile;
     if (epi != Epi::RowScale || wk == WKind::U4Asym) return false;
     // Every kernel sums int32 exactly, so the quicker one takes the product. Many columns and rows:
     // the wide kernel's 128 x 128 tiles share each operand over more products than the few-row
@@ -306,7 +307,7 @@ bool gemm_runs_wide(const GemmArgs& a, WKind wk, Epi epi) {
         (wk != WKind::U4Asym || a.wtile || (a.ldwz % 2 == 0 && reinterpret_cast<uintptr_t>(a.wz) % 2 == 0)) &&
         (epi != Epi::GroupScale || (a.ldws % 2 == 0 && reinterpret_cast<uintptr_t>(a.ws16) % 4 == 0));
     // (K >= 192: the wide kernel's last-row load correction needs at least three K groups)
-    // Weights in 16-row tiles are read by the wide kernel at every M above the GEMV's few rows.
+    // Weights in 16-row tiles are read here at every M that the GEMV and the few-row kernel leave.
     return (a.M > 128 || a.wtile) && a.K >= 192 && fits32 && zs_aligned && a.act_mode != 1;
 }
 

@@ -1,5 +1,6 @@
-// Quantized GEMM for a few activation rows (5 <= M <= 128: a text prompt's tokens, a small batch of
-// modulation vectors) with the scaled epilogues, GroupScale and RowScale.
+// Quantized GEMM for a few activation rows (5 <= M <= 128, or fewer that are too long for the GEMV's LDS: a
+// text prompt's tokens, a small batch of modulation vectors) with the scaled epilogues, GroupScale and
+// RowScale.
 //
 // What bounds it: at these sizes the product is a read of the weights (4.7 MB packed at
 // N = K = 3072) with far too few output tiles to fill 256 compute units, so the work is split along

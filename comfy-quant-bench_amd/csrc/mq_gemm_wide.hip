@@ -277,8 +277,11 @@ __device__ __forceinline__ T& lds(uint8_t* smem, int off) {
 // NS: stages of the LDS ring. Eight for the 128 x 128 tile's int8 row-scale products when every compute
 // unit has at most one workgroup: their groups are short (eight MFMAs per wave and nothing else), so
 // four stages give the DMA of a group, two groups' time to arrive, less than its latency. W8A8 linears,
-// us, 4 -> 8 stages: 256 x 3072 x 3072 18.9 -> 16.5, 200 x 4000 x 3072 18.7 -> 16.6, 256 x 12288 x 3072
-// 21.0 -> 19.8, 1024 x 3072 x 3072 23.6 -> 22.6. The group-scale products, bound by the VALU and LDS work
+// us back to back, 4 -> 8 stages: 256 x 3072 x 3072 18.0 -> 16.6, 200 x 4000 x 3072 17.5 -> 16.3, 256 x 12288 x 3072
+// 20.1 -> 18.2, 1024 x 3072 x 3072 21.6 -> 19.3 (a slower clock gave 21.0 -> 19.8 for the third). Split along K,
+// every slice but the last fetches seven groups of its neighbour's that it does not use, where four
+// stages fetch three; split products gain all the same: 256 x 3072 x 12288 30.5 -> 29.6, 400 x 3072 x 12288 44.3 ->
+// 38.7, 256 x 1024 x 12288 28.2 -> 27.6. The group-scale products, bound by the VALU and LDS work
 // of their groups, gain nothing (1024 x 3072 x 3072 30.3 -> 31.0) and keep four; so do larger launches,
 // which fit two such workgroups' LDS on a compute unit.
 template <int TM_, int TN_, WKind WK, Epi EPI, int AM, bool SPLIT, bool XP, int NS>

@@ -101,8 +101,9 @@ struct GemmArgs {
     // 4-bit kind (group scales): the weights expanded to int8 in those tiles (mq_expand_weight_w4),
     // read by the wide kernel only; wz then only tells uint4 asymmetric (non-null) from signed
     int wtile = 0;
-    // activation codes (qa) in the same 16-row tiles, [ceil(M / 16)][K / 64][16][64] (lda = K):
-    // written so by the whole-linear entries when the wide kernel runs their product
+    // activation codes (qa) in the same 16-row tiles, [ceil(M / 16)][K / 64][16][64] (lda = K): written
+    // so by the whole-linear entries when the wide or few-row kernel runs their product. The last band
+    // is 16 rows whatever M is: the few-row kernel reads its rows past M (and drops what they give)
     int atile = 0;
     // One-row whole linears (gemv_quantizes_row): the GEMV rotates and quantizes the activation
     // row x (x_dtype, Hadamard block hblock, x_bits-bit codes) itself instead of reading qa / sa
@@ -143,7 +144,7 @@ __host__ __device__ inline int group_shift(int act_mode, WKind wk) {
 }
 
 int launch_gemm(const GemmArgs& a, WKind wk, Epi epi, hipStream_t stream);
-// whether launch_gemm runs these arguments' product on the wide kernel (the one that reads atile)
+// whether launch_gemm runs these arguments' product on the wide kernel (it and the few-row one read atile)
 bool gemm_runs_wide(const GemmArgs& a, WKind wk, Epi epi);
 
 // M <= 4 rows, GroupScale / RowScale only (mq_gemv.hip).
@@ -153,8 +154,9 @@ int launch_gemv(const GemmArgs& a, WKind wk, Epi epi, hipStream_t stream);
 // the rotate+quantize kernel's arithmetic, in the same launch.
 bool gemv_quantizes_row(const GemmArgs& a, WKind wk, Epi epi);
 
-// 5 <= M <= 128 rows, GroupScale / RowScale (mq_gemm_few.hip); whether launch_gemm runs these
-// arguments' product there (it reads qa in rows or in 16-row tiles).
+// Up to 128 rows that the GEMV does not take (M >= 5, or M * K > 131072), GroupScale / RowScale
+// (mq_gemm_few.hip); whether launch_gemm runs these arguments' product there (it reads qa in rows or in
+// 16-row tiles).
 int launch_gemm_few(const GemmArgs& a, WKind wk, Epi epi, hipStream_t stream);
 bool gemm_runs_few(const GemmArgs& a, WKind wk, Epi epi);
 

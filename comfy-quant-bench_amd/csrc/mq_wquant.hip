@@ -6,8 +6,8 @@
 // experiments/qwen21-kernel/kernels/g64_quant.cu:68-86 in registers and an LDS transpose). The group
 // formats need nothing across chunks (a 64-column group is four lanes of one 16-lane row), so every
 // wave takes one chunk of one row and nothing waits at a barrier; the row formats give a row to the
-// four waves of a workgroup, NCH chunks each, which combine the row's maximum through LDS. With
-////   U4_ASYM_G64  lo = min(min w, 0), hi = max(max w, 0), s = fp16((hi - lo) / 15),
+// four waves of a workgroup, NCH chunks each, which combine the row's maximum through LDS. The formats:
+//   U4_ASYM_G64  lo = min(min w, 0), hi = max(max w, 0), s = fp16((hi - lo) / 15),
 //                z = clamp(rne(-lo / s), 0, 15), q = clamp(rne(w / s) + z, 0, 15); s = 0 -> q = z = 0
 //   I4_SYM_G64   s = fp16(max |w| / 7), q = clamp(rne(w / s), -7, 7); s = 0 -> q = 0
 //   I4_ROW       s = max(max |w|, 1e-10) / 7,   q = clamp(rne(w / s), -7, 7)
@@ -337,8 +337,9 @@ __global__ void __launch_bounds__(256) tile16_kernel(const uint8_t* w, int64_t l
 // weights: (q + 0x80 - z) ^ 0x80 per byte, or (0x80 + z - q) ^ 0x80 negated, without inter-byte carries,
 // and two byte permutes back to k order: about two operations a value where the value at a time it
 // replaces, bound by its VALU work, took six and two 64-bit divisions a thread (the expansion is under 2 GiB, so
-// the tiles count in 32 bits and the division is one per wave). With the scales' launch below, [12288, 3072] uint4 takes 18-19.5 us (26.4 before;
-// its 60 MB take 12 at the rate of a large copy), [3072, 14336] 18.4 (28.7), row-scale [3072, 12288] 11.4 (19.4).
+// the tiles count in 32 bits and the division is one per wave). expand_w4_weight, calls back to back, with the scales' launch below:
+// [12288, 3072] uint4 15.9 us (22.9 before; its 60 MB take 12 at the rate of a large copy), [3072, 14336] 16.8
+// (25.9); row-scale [3072, 12288] 10.0 (17.6).
 enum ExpandKind : int { kExpandU4 = 0, kExpandI4 = 1, kExpandI4x16 = 2 };
 template <int KIND>
 __global__ void __launch_bounds__(64 * kWaves)

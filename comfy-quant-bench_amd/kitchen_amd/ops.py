@@ -422,11 +422,11 @@ def expand_w4_weight(qweight: torch.Tensor, wzeros=None, layout: int = _lib.ACT_
     return ExpandedW4(buf, layout, zz is not None, n, k, None if ws is None else _scales_id(ws))
 
 
-# The linears run their 4-bit weights from an int8 expansion wherever the packed weights would run
-# on the wide kernel too, so that the results are the same bits either way: group scales above 128
-# rows (fewer rows run on the few-row kernel, whose group epilogue rounds differently),
-# row scales above the GEMV's 4 rows (exact int32 sums on every kernel). The GEMV reads the packed
-# bytes: it is bound by their HBM traffic. The expansion is made on a weight's first such call and
+# The linears run their 4-bit weights from an int8 expansion wherever the results are the same bits
+# either way: group scales above 128 rows, where the packed weights run on the wide kernel too (fewer rows
+# run on the few-row kernel, whose group epilogue rounds differently), row scales above the GEMV's 4
+# rows (exact int32 sums on every kernel; up to 128 rows most run on the few-row kernel, which reads
+# either form). The GEMV reads the packed bytes: it is bound by their HBM traffic. The expansion is made on a weight's first such call and
 # kept until the tensor it was made from (its base tensor, for a view) is freed, for as long as that
 # weight's storage and version are unchanged; it costs 1 byte per weight element beside the packed
 # 0.5 (release_expanded_weights() drops them all). A HIP graph that captured a linear keeps the

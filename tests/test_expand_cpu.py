@@ -12,7 +12,7 @@ def _w(n=256, k=3072):
 def test_expansion_only_where_the_wide_kernel_reads_it():
     w = _w()
     s = torch.zeros((256, 48), dtype=torch.float16)
-    # group scales: the packed weights' few rows (<= 128) run on the 128 x 128 kernel, whose
+    # group scales: the packed weights' few rows (<= 128) run on the few-row kernel, whose
     # epilogue rounds differently, so they keep the packed weights (the same bits either way)
     for m in (1, 4, 5, 128):
         assert ops._expansion(w, None, _lib.ACT_I8, m, 3072, s) is None

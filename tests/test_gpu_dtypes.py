@@ -140,8 +140,8 @@ def _round_to(y32: np.ndarray, dt) -> np.ndarray:
 @pytest.mark.parametrize("bias_dtype", [None, torch.bfloat16, torch.float16, torch.float32])
 def test_rowscale_output_types_exact(gpu_device, m, bias_dtype):
     # exact int32 sums, so every kernel's output is the fp32 expression ((acc * sa) * ws) + bias
-    # rounded to the output type, bit for bit: M = 1 / 3 the few-row kernel, 77 the 128-tile
-    # kernel, 256 the split-K wide kernel, 1000 the wide kernel
+    # rounded to the output type, bit for bit: M = 1 / 3 the GEMV, 77 the few-row kernel,
+    # 256 the split-K wide kernel, 1000 the wide kernel
     n, k = 640, 3072
     rng = np.random.default_rng(m)
     qa = rng.integers(-127, 128, (m, k)).astype(np.int8)

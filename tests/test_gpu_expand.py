@@ -107,7 +107,7 @@ def test_group_gemm_expanded_equals_packed(gpu_device, m, n, k, act_mode, asym):
     if m > ops.FEW_ROWS:
         assert torch.equal(y, y0)
     else:
-        # the packed weights' few rows run on the 128 x 128 kernel (int32 partials converted, then one
+        # the packed weights' few rows run on the few-row kernel (int32 partials converted, then one
         # fp32 fma per group): the same exact partials, summed in fp32 in another order, so the
         # outputs agree to within a rounding step of the output type
         assert torch.allclose(y.float(), y0.float(), rtol=2 ** -7, atol=2e-2)

@@ -97,3 +97,20 @@ def test_linears_read_tiles_as_rows(gpu_device, m, n, k, pad):
     y4 = ops.gemm_rowscale(qa, sa, ops.tile_int8_weight(w8), sw, None, n, 8)
     torch.cuda.synchronize()
     assert torch.equal(y3.view(torch.int16), y4.view(torch.int16))
+
+
+@pytest.mark.parametrize("m,k", [(1, 32768 * 4 + 64), (2, 65536), (3, 43776), (4, 32832), (4, 65600)])
+def test_rows_past_the_gemv(gpu_device, m, k):
+    """One to four rows that the GEMV's LDS does not hold (M * K > 131072): the few-row kernel to K = 65536, the
+    128 x 128-tile kernel past it."""
+    n = 48
+    print(f"[few] long rows M={m} K={k}", flush=True)
+    rng = np.random.default_rng(m + k)
+    qa = rng.integers(-127, 128, (m, k)).astype(np.int8)
+    qw = rng.integers(-127, 128, (n, k)).astype(np.int8)
+    sa, sw = rng.uniform(0.01, 0.02, m).astype(np.float32), rng.uniform(0.001, 0.002, n).astype(np.float32)
+    y = ops.gemm_rowscale(_t(qa, gpu_device), _t(sa, gpu_device), _t(qw, gpu_device), _t(sw, gpu_device), None, n, 8,
+                          out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    p = gemm.partials(qa, qw, k)[0].astype(np.float32)
+    assert np.array_equal(y.cpu().numpy(), (p * sa[:, None]) * sw)

@@ -116,8 +116,8 @@ def test_rowscale_acc_and_output(gpu_device, wbits, m, n, k):
 
 
 # ---------------------------------------------------------------- activation layouts and tile paths
-# M <= 128 runs the few-row 128 x 128-tile kernel; larger M the wide kernel, on 128 x 128 tiles for
-# small products and 256 x 256 or 256 x 192 tiles for large ones: all are covered.
+# M <= 128 runs the few-row kernel (its partials entry the 128 x 128-tile one); larger M the wide
+# kernel, on 128 x 128 tiles for small products and 256 x 256 or 256 x 192 tiles for large ones: all are covered.
 
 def _x16alt(qa):
     """The group GEMM's int4 operand layout (mq_rotquant MQ_Q_X16ALT): 16 * q, odd groups negated."""
