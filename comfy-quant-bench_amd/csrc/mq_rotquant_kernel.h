@@ -405,7 +405,9 @@ int launch_rq(const uint16_t* x, int64_t M, int64_t K, int64_t ldx, void* q, int
     }
     if (wgs == 0) return 0;
     const bool nt = (OUT == 2 ? M * K / 2 : M * K) >= kNtCodeBytes;
-    constexpr bool kDead = W > 1 && !(ACT >= 1 && IN == 1);   // (nothing is gained where the gathers set the time)
+    // (fp16 SwiGLU, whose gathers set the time: with four chunks a wave only, us: M = 4096, K = 14336 119.7 -> 116.5,
+    // but K = 9216 76.7 -> 77.5 and K = 5120 43.3 -> 44.4)
+    constexpr bool kDead = W > 1 && !(ACT >= 1 && IN == 1 && NCH < 4);
     const bool dead = kDead && K <= (NCH * W - 1) * 1024;
     // a row stride of 0 asks for the codes in 16-row tiles (one code per byte)
     const bool tiled = OUT != 2 && ldq == 0;
