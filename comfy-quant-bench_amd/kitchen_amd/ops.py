@@ -451,8 +451,8 @@ class _Ready:
         self.tensors, self.streams = tensors, {stream}
 
     def on(self, device, stream: int) -> None:
-        """Before a launch on `stream`, torch's current stream on `device`."""
-        if stream in self.streams or torch.cuda.is_current_stream_capturing():
+        """Before a launch on `stream`, torch's current stream on `device`, which is not among `streams`."""
+        if torch.cuda.is_current_stream_capturing():
             return
         torch.cuda.synchronize(device)
         for t in self.tensors:
@@ -484,7 +484,8 @@ def _expansion(qweight, wzeros, layout: int, m: int, k: int, wscales=None, strea
     per = _EXPANDED.get(id(root))
     hit = None if per is None else per.get(key)
     if hit is not None and hit[0] == sig:
-        hit[2].on(qweight.device, stream)
+        if stream not in hit[2].streams:
+            hit[2].on(qweight.device, stream)
         return hit[1]
     if torch.cuda.is_current_stream_capturing():
         return None   # nothing is allocated under capture: the packed weights, unless expanded before
@@ -597,14 +598,6 @@ def _linear_input(x: torch.Tensor, swiglu: int, k: int):
     return x2, swiglu
 
 
-def _output(x2: torch.Tensor, m: int, n: int, out_dtype) -> torch.Tensor:
-    """A linear's output [M, N] on x2's device: a plain tensor whatever x2's class (new_empty, which keeps
-    the class, is the cheaper call: one-row linears are bound by their host time)."""
-    if type(x2) is not torch.Tensor:
-        return torch.empty((m, n), dtype=out_dtype, device=x2.device)
-    return x2.new_empty((m, n)) if out_dtype is x2.dtype else x2.new_empty((m, n), dtype=out_dtype)
-
-
 def _linear_w4_group(x, swiglu, cg, act_bits, qweight, wscales, wzeros, bias, n, k, out_dtype):
     """rotate + quantize + group GEMM in one library call (mq_linear_w4_group)."""
     x2, swiglu = _linear_input(x, swiglu, k)
@@ -612,7 +605,9 @@ def _linear_w4_group(x, swiglu, cg, act_bits, qweight, wscales, wzeros, bias, n,
     _check_w4_group_weights(qweight, wscales, wzeros, n, k, INT4_GROUP_SIZE)
     dev = x2.device
     b = _bias(bias, n, dev)
-    y = _output(x2, m, n, out_dtype)
+    # a plain tensor whatever x2's class (new_empty keeps the class; it is the cheaper call)
+    y = torch.empty((m, n), dtype=out_dtype, device=dev) if type(x2) is not torch.Tensor else \
+        x2.new_empty((m, n)) if out_dtype is x2.dtype else x2.new_empty((m, n), dtype=out_dtype)
     if m == 0:
         return y
     stream = _lib.stream_of_device(dev)
@@ -654,7 +649,9 @@ def _linear_rowscale(x, swiglu, cg, act_bits, qweight, wbits, wscales, bias, n, 
             qw, wbits, tiles = xw.tiles, 8, True
     ldw, wbits = _weight_args(qw, n, k, wbits) if tiles else (wbytes, wbits)
     b = _bias(bias, n, dev)
-    y = _output(x2, m, n, out_dtype)
+    # a plain tensor whatever x2's class (new_empty keeps the class; it is the cheaper call)
+    y = torch.empty((m, n), dtype=out_dtype, device=dev) if type(x2) is not torch.Tensor else \
+        x2.new_empty((m, n)) if out_dtype is x2.dtype else x2.new_empty((m, n), dtype=out_dtype)
     if m == 0:
         return y
     work = _linear_workspace(m, n, k, dev, stream)
@@ -678,7 +675,9 @@ def _decoded_w4a8(qdata, s_rel, s_channel, codebook, group_size):
     qid = id(qdata)
     hit = _DECODED.get(qid)
     if hit is not None and hit[0] == sig:
-        hit[2].on(qdata.device, _lib.stream_of(qdata))
+        stream = _lib.stream_of(qdata)
+        if stream not in hit[2].streams:
+            hit[2].on(qdata.device, stream)
         return hit[1]
     dec = decode_w4a8_codebook_weight(qdata, s_rel, s_channel, codebook, group_size)
     if hit is None:
